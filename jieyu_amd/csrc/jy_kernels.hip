@@ -139,8 +139,56 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ 
     block_rmsnorm(xr, n, w, Y + (size_t)blockIdx.x * n, red);
 }
 
+// The same with the row and the weights in registers (NV float4s per thread, n a multiple
+// of 4 and at most 1024 NV): every load goes out at once, so the kernel waits for memory
+// once and not once per 256 elements; the same arithmetic element by element.
+// One row of 4096: 14.8 us before, with the chain of block_rms_scale.
+template <int NV>
+__global__ __launch_bounds__(256) void rmsnorm4_kernel(const float* __restrict__ X, float* __restrict__ Y,
+                                                       const float* __restrict__ w, int n) {
+    extern __shared__ __align__(16) float xr[];
+    __shared__ float red[18];
+    const float4* x4 = reinterpret_cast<const float4*>(X + (size_t)blockIdx.x * n);
+    const float4* w4 = reinterpret_cast<const float4*>(w);
+    float4* y4 = reinterpret_cast<float4*>(Y + (size_t)blockIdx.x * n);
+    const int n4 = n / 4;
+    float4 v[NV], wv[NV];
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = threadIdx.x + 256 * j;
+        v[j] = i < n4 ? x4[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        wv[j] = i < n4 ? w4[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = threadIdx.x + 256 * j;
+        if (i < n4) reinterpret_cast<float4*>(xr)[i] = v[j];
+    }
+    __syncthreads();
+    block_rms_scale(xr, n, red);
+    const float scale = red[16];
+    const bool zero = red[17] != 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = threadIdx.x + 256 * j;
+        if (i < n4)
+            y4[i] = zero ? make_float4(0.0f, 0.0f, 0.0f, 0.0f)
+                         : make_float4((v[j].x * scale) * wv[j].x, (v[j].y * scale) * wv[j].y,
+                                       (v[j].z * scale) * wv[j].z, (v[j].w * scale) * wv[j].w);
+    }
+}
+
 void launch_rmsnorm(const float* X, float* Y, const float* w, int n, int rows, hipStream_t st) {
-    hipLaunchKernelGGL(rmsnorm_kernel, dim3(rows), dim3(256), (size_t)n * sizeof(float), st, X, Y, w, n);
+    const size_t lds = (size_t)n * sizeof(float);
+    // (rows and weights come from device allocations: 16-byte aligned when n is a multiple of 4)
+    if (n % 4 == 0 && n <= 1024)
+        hipLaunchKernelGGL(rmsnorm4_kernel<1>, dim3(rows), dim3(256), lds, st, X, Y, w, n);
+    else if (n % 4 == 0 && n <= 4096)
+        hipLaunchKernelGGL(rmsnorm4_kernel<4>, dim3(rows), dim3(256), lds, st, X, Y, w, n);
+    else if (n % 4 == 0 && n <= 8192)
+        hipLaunchKernelGGL(rmsnorm4_kernel<8>, dim3(rows), dim3(256), lds, st, X, Y, w, n);
+    else
+        hipLaunchKernelGGL(rmsnorm_kernel, dim3(rows), dim3(256), lds, st, X, Y, w, n);
 }
 
 // ---------------------------------------------------------------- dense matvec (decode, [K][N] weights)

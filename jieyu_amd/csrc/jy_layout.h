@@ -80,32 +80,61 @@ __device__ __forceinline__ float kq_elem(const KQDev& W, int R, int k) {
 // y = (x*scale)*w.  red: 18 floats of shared memory.
 // The scale part: red[16] = 1/sqrtf(den), red[17] = 1 where den <= 0 (the row then
 // normalises to zeros); both visible to the whole workgroup on return.
+//
+// What bounds it is the chain of n/16 dependent FMAs per lane.  The LDS reads run one
+// batch of RMS_G steps ahead of the FMAs in a second register set; with one batch read
+// and then consumed, every step paid LDS latency.
+static constexpr int RMS_G = 16;
 __device__ __forceinline__ void block_rms_scale(const float* x, int n, float* red) {
     const int t = threadIdx.x;
     const int n16 = n / 16 * 16;
     const bool rem8 = n16 + 8 <= n;
-    if (t < 16) {
+    if (t < 64) {  // (lanes 16..63 repeat lanes 0..15's chains: the wave stays converged)
+        const int l = t & 15;
+        const int steps = n16 / 16, nb = steps / RMS_G;
+        const float* xl = x + l;
         float a = 0.0f;
-#pragma unroll 8
-        for (int i = t; i < n16; i += 16) a = __builtin_fmaf(x[i], x[i], a);
-        if (t < 8 && rem8) a = __builtin_fmaf(x[n16 + t], x[n16 + t], a);
-        red[t] = a;
-    }
-    __syncthreads();
-    if (t == 0) {
-        float s[8], q[4];
+        float va[RMS_G], vb[RMS_G];
+        // batch b (clamped to the last full one: always a read inside the row)
+        auto rd = [&](float(&v)[RMS_G], int b) {
+            const float* p = xl + min(b, nb - 1) * (16 * RMS_G);
 #pragma unroll
-        for (int l = 0; l < 8; l++) s[l] = red[l] + red[8 + l];
+            for (int i = 0; i < RMS_G; i++) v[i] = p[16 * i];
+        };
+        auto fm = [&](const float(&v)[RMS_G]) {
 #pragma unroll
-        for (int l = 0; l < 4; l++) q[l] = s[l] + s[4 + l];
-        float ss = (q[0] + q[1]) + (q[2] + q[3]);
-        int i = n16 + (rem8 ? 8 : 0);
-        if (n - i >= 4)
-            for (const int e = i + 4; i < e; i++) ss = ss + x[i] * x[i];
-        for (; i < n; i++) ss = __builtin_fmaf(x[i], x[i], ss);
-        const float den = ss / (float)n + 1e-5f;
-        red[17] = den <= 0.0f ? 1.0f : 0.0f;
-        red[16] = den <= 0.0f ? 0.0f : 1.0f / sqrtf(den);
+            for (int i = 0; i < RMS_G; i++) a = __builtin_fmaf(v[i], v[i], a);
+        };
+        if (nb > 0) {
+            rd(va, 0);
+            int b = 0;
+            for (; b + 1 < nb; b += 2) {
+                rd(vb, b + 1);
+                __builtin_amdgcn_sched_barrier(0);  // the next batch's reads stay ahead of the FMAs
+                fm(va);
+                rd(va, b + 2);
+                __builtin_amdgcn_sched_barrier(0);
+                fm(vb);
+            }
+            if (b < nb) fm(va);
+        }
+        for (int i = nb * RMS_G; i < steps; i++) a = __builtin_fmaf(xl[16 * i], xl[16 * i], a);
+        if (l < 8 && rem8) a = __builtin_fmaf(x[n16 + l], x[n16 + l], a);
+        // the fold as butterflies: every add of the tree is commutative, so lane 0 ends with
+        // the reference's value bit for bit
+        float s = a + dpp_f<0x128>(a);   // s[i] = v[i] + v[8+i]
+        s = s + dpp_f<0x12C>(s);         // q[i] = s[i] + s[4+i]
+        s = s + dpp_f<0xB1>(s);          // q0+q1 (lane 0), q2+q3 (lane 2)
+        float ss = s + dpp_f<0x4E>(s);   // (q0+q1) + (q2+q3)
+        if (t == 0) {
+            int i = n16 + (rem8 ? 8 : 0);
+            if (n - i >= 4)
+                for (const int e = i + 4; i < e; i++) ss = ss + x[i] * x[i];
+            for (; i < n; i++) ss = __builtin_fmaf(x[i], x[i], ss);
+            const float den = ss / (float)n + 1e-5f;
+            red[17] = den <= 0.0f ? 1.0f : 0.0f;
+            red[16] = den <= 0.0f ? 0.0f : 1.0f / sqrtf(den);
+        }
     }
     __syncthreads();
 }
