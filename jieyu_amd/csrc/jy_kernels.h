@@ -292,6 +292,14 @@ void launch_repack_kq(const uint8_t* src, const KQDev& dst, hipStream_t st);
 // quantized rows, fma chain over k for dense [in][out]); EPI_STORE / EPI_BIAS /
 // EPI_RESID
 void launch_mv(const DevW& W, const float* x, float* out, Epi epi, const float* aux, hipStream_t st);
+// The same with the input's RMSNorm (norm weights nw) in the launch, for k-quant matrices of
+// at most 8192 inputs; each returns false, having launched nothing, where it does not apply:
+//   launch_mv_norm     out = W norm(x)
+//   launch_mv_qkv      W[0..2] = q, k, v: the rows (+ a.aux) with q and k rotated (EPI_ROPE)
+//   launch_mv_gate_up  h = silu(gate norm(x)) * (up norm(x)), both of one type
+bool launch_mv_norm(const DevW& W, const float* x, const float* nw, float* out, hipStream_t st);
+bool launch_mv_qkv(const DevW* W, const float* x, const float* nw, float* qkv, const MvArgs& a, hipStream_t st);
+bool launch_mv_gate_up(const DevW& gate, const DevW& up, const float* x, const float* nw, float* h, hipStream_t st);
 // C[i][j] (row stride ldc) for m > 1 rows: the generic quantized path (product and
 // sum rounded apart, k ascending) or the dense fma chain
 void launch_gemm(const DevW& W, int m, const float* A, float* C, int ldc, const float* aux, Epi epi,

@@ -136,7 +136,7 @@ __device__ __forceinline__ void block_rms_scale(const float* x, int n, float* re
             red[16] = den <= 0.0f ? 0.0f : 1.0f / sqrtf(den);
         }
     }
-    __syncthreads();
+    lds_barrier();  // (only LDS is ordered: a caller's loads stay in flight)
 }
 
 __device__ __forceinline__ void block_rmsnorm(const float* x, int n, const float* __restrict__ w,

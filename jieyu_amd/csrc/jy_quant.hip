@@ -10,7 +10,7 @@
 // (two lanes each), 4 rows per wave, the activation vector lane-pair major in LDS.
 #include <algorithm>
 
-#include "jy_layout.h"
+#include "jy_matvec.h"
 
 namespace jy {
 
@@ -160,70 +160,44 @@ __device__ __forceinline__ void kq_chunk(const uint2& nb, uint32_t hb, const uin
     }
 }
 
-static constexpr int KQ_U = 4;  // chunks per register buffer (two buffers)
+// The chunk stream of one wave's row groups in registers: U chunks of one matrix.
+template <int TYPE, int U>
+struct KqBuf {
+    uint2 nb[U];
+    uint32_t hb[U];
+    uint4 h[U];
+    uint32_t dm[U];
 
-// one row group per wave, 4 waves per workgroup
-template <int TYPE, int EPI>
-__global__ __launch_bounds__(256) void matvec_kq_kernel(KQDev W, const float* __restrict__ x, float* __restrict__ out,
-                                                        const float* __restrict__ aux) {
-    extern __shared__ __align__(16) float xs[];  // [16][XS]: lane pair g, 16 floats per chunk
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int r = lane >> 4, g = lane & 15;
-    const int K = W.cols, nsb = W.nsb, XS = 16 * nsb + 4;
-    for (int k = tid; k < K; k += blockDim.x) xs[((k & 31) >> 1) * XS + 2 * (k >> 5) + (k & 1)] = x[k];
-    __syncthreads();
-    const int rg = blockIdx.x * 4 + wave;
-    if (rg >= W.groups) return;
-    const float* xrow = xs + g * XS;
-    float a0 = 0.0f, a1 = 0.0f;
-    const size_t c0 = (size_t)rg * nsb;
-    // two buffers of KQ_U chunks: the next buffer's loads are in flight while the
-    // current one is computed (chunk indices past the row clamp to its last chunk)
-    struct Buf {
-        uint2 nb[KQ_U];
-        uint32_t hb[KQ_U];
-        uint4 h[KQ_U];
-        uint32_t dm[KQ_U];
-    };
-    auto load = [&](Buf& b, int s0) {
+    // chunks s0 .. s0 + U - 1 of row group rg (indices past the row clamp to its last
+    // chunk: read, never used)
+    __device__ __forceinline__ void load(const KQDev& W, int rg, int s0, int lane, int r) {
 #pragma unroll
-        for (int u = 0; u < KQ_U; u++) {
-            const size_t c = c0 + min(s0 + u, nsb - 1);
-            b.nb[u] = *reinterpret_cast<const uint2*>(W.nib + (c * 64 + lane) * 8);
-            b.hb[u] = TYPE == JY_Q5_K   ? *reinterpret_cast<const uint16_t*>(W.hi + (c * 64 + lane) * 2)
-                      : TYPE == JY_Q6_K ? *reinterpret_cast<const uint32_t*>(W.hi + (c * 64 + lane) * 4)
-                                        : 0u;
-            b.h[u] = *reinterpret_cast<const uint4*>(W.hdr + c * 64 + r * 16);
-            b.dm[u] = W.dm[c * 4 + r];
+        for (int u = 0; u < U; u++) {
+            const size_t c = (size_t)rg * W.nsb + min(s0 + u, W.nsb - 1);
+            nb[u] = *reinterpret_cast<const uint2*>(W.nib + c * 512 + lane * 8);
+            hb[u] = TYPE == JY_Q5_K   ? *reinterpret_cast<const uint16_t*>(W.hi + c * 128 + lane * 2)
+                    : TYPE == JY_Q6_K ? *reinterpret_cast<const uint32_t*>(W.hi + c * 256 + lane * 4)
+                                      : 0u;
+            h[u] = *reinterpret_cast<const uint4*>(W.hdr + c * 64 + r * 16);
+            dm[u] = W.dm[c * 4 + r];
         }
-    };
-    auto compute = [&](const Buf& b, int s0) {
-#pragma unroll
-        for (int u = 0; u < KQ_U; u++) {
-            if (s0 + u < nsb) {
-                float xv[16];
-                const float4* xp = reinterpret_cast<const float4*>(xrow + 16 * (s0 + u));
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const float4 v = xp[q];
-                    xv[4 * q] = v.x;
-                    xv[4 * q + 1] = v.y;
-                    xv[4 * q + 2] = v.z;
-                    xv[4 * q + 3] = v.w;
-                }
-                kq_chunk<TYPE>(b.nb[u], b.hb[u], b.h[u], b.dm[u], g, xv, a0, a1);
-            }
-        }
-    };
-    Buf A, B;
-    load(A, 0);
-    for (int s0 = 0; s0 < nsb; s0 += 2 * KQ_U) {
-        load(B, s0 + KQ_U);
-        compute(A, s0);
-        if (s0 + 2 * KQ_U < nsb) load(A, s0 + 2 * KQ_U);
-        compute(B, s0 + KQ_U);
     }
-    // lanes 2g, 2g+1 -> the reference's reduction tree (as in the Q8_0 matvec)
+};
+
+__device__ __forceinline__ void kq_x(const float* xrow, int s, float* xv) {
+    const float4* xp = reinterpret_cast<const float4*>(xrow + 16 * s);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const float4 v = xp[q];
+        xv[4 * q] = v.x;
+        xv[4 * q + 1] = v.y;
+        xv[4 * q + 2] = v.z;
+        xv[4 * q + 3] = v.w;
+    }
+}
+
+// lanes 2g, 2g+1 -> the reference's reduction tree (as in the Q8_0 matvec)
+__device__ __forceinline__ float kq_tree(float a0, float a1) {
     a0 += dpp_f<0x12C>(a0);
     a1 += dpp_f<0x12C>(a1);
     a0 += dpp_f<0x128>(a0);
@@ -231,24 +205,324 @@ __global__ __launch_bounds__(256) void matvec_kq_kernel(KQDev W, const float* __
     a0 += dpp_f<0x4E>(a0);
     a1 += dpp_f<0x4E>(a1);
     const float t = a0 + a1;
-    const float y = t + dpp_f<0xB1>(t);
-    const int row = rg * 4 + r;
-    if (g == 0 && row < W.rows) {
-        if (EPI == EPI_STORE) out[row] = y;
-        if (EPI == EPI_BIAS) out[row] = y + aux[row];
-        if (EPI == EPI_RESID) out[row] = out[row] + y;
+    return t + dpp_f<0xB1>(t);
+}
+
+// x (K floats) into LDS in lane-pair order, `pre()` (the first weight loads) issued once x's
+// first loads are out.  With NORM the RMSNorm comes first: x and the norm weights stay in
+// registers (NV float4s per thread: K <= 1024 NV; NV = 0: no norm, SB
+// float4s per thread at a time), x goes to LDS in its own order for the sum of squares, then
+// (x * scale) * w in lane-pair order over it.  Only LDS is ordered by the barriers, so the
+// weight loads stay in flight.
+static constexpr int KQ_NORM_MAX = 8192;
+template <int NV, int SB, class Pre>
+__device__ __forceinline__ void kq_stage(const float* __restrict__ x, const float* __restrict__ nw, int K, int XS,
+                                         float* xs, float* red, Pre&& pre) {
+    const int tid = threadIdx.x, n4 = K / 4;
+    const float4* x4 = reinterpret_cast<const float4*>(x);
+    auto put = [&](int i, float4 v) {
+        xs[xs_index(4 * i, XS)] = v.x;
+        xs[xs_index(4 * i + 1, XS)] = v.y;
+        xs[xs_index(4 * i + 2, XS)] = v.z;
+        xs[xs_index(4 * i + 3, XS)] = v.w;
+    };
+    if constexpr (NV > 0) {
+        const float4* w4 = reinterpret_cast<const float4*>(nw);
+        float4 v[NV], wv[NV];
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+            const int i = tid + 256 * j;
+            v[j] = i < n4 ? x4[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            wv[j] = i < n4 ? w4[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+        pre();
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+            const int i = tid + 256 * j;
+            if (i < n4) reinterpret_cast<float4*>(xs)[i] = v[j];
+        }
+        lds_barrier();
+        block_rms_scale(xs, K, red);
+        const float scale = red[16];
+        const bool zero = red[17] != 0.0f;
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+            const int i = tid + 256 * j;
+            if (i < n4)
+                put(i, zero ? make_float4(0.0f, 0.0f, 0.0f, 0.0f)
+                            : make_float4((v[j].x * scale) * wv[j].x, (v[j].y * scale) * wv[j].y,
+                                          (v[j].z * scale) * wv[j].z, (v[j].w * scale) * wv[j].w));
+        }
+    } else {
+        for (int b0 = 0; b0 < n4; b0 += SB * 256) {
+            float4 v[SB];
+#pragma unroll
+            for (int j = 0; j < SB; j++) {
+                const int i = b0 + tid + 256 * j;
+                v[j] = i < n4 ? x4[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+            if (b0 == 0) pre();
+#pragma unroll
+            for (int j = 0; j < SB; j++) {
+                const int i = b0 + tid + 256 * j;
+                if (i < n4) put(i, v[j]);
+            }
+        }
+    }
+    lds_barrier();
+}
+
+// Up to three k-quant matrices of the same input in one launch (q, k and v), each with
+// workgroups of its own; rows are numbered through them (row0).
+struct KqMats {
+    KQDev W[3];
+    int wg0[4];   // first workgroup of each matrix, then the total
+    int row0[3];  // first output row of each matrix
+};
+
+// One matrix by `nwg` workgroups of 4 waves: wave w takes row groups w, w + 4 nwg, ...
+template <int TYPE, int EPI, int NV, int U>
+__device__ __forceinline__ void kq_body(const KQDev& W, int wg, int nwg, int row0, const float* __restrict__ x,
+                                        const float* __restrict__ nw, float* __restrict__ out, const MvArgs& a,
+                                        float* xs, float* red) {
+    const int lane = threadIdx.x & 63, r = lane >> 4, g = lane & 15;
+    const int wid = wg * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), TW = nwg * 4;
+    const int nsb = W.nsb, XS = 16 * nsb + 4;
+    // two buffers of U chunks, two ahead of the compute, across row groups
+    KqBuf<TYPE, U> A, B;
+    int lrg = min(wid, W.groups - 1), lp = 0;  // row group and chunk of the next load
+    auto load = [&](KqBuf<TYPE, U>& b) {
+        b.load(W, lrg, lp, lane, r);
+        lp += U;
+        if (lp >= nsb) {
+            lp = 0;
+            lrg = min(lrg + TW, W.groups - 1);
+        }
+    };
+    kq_stage<NV, U>(x, nw, W.cols, XS, xs, red, [&]() {
+        load(A);
+        if (NV == 0) load(B);
+    });
+    if (NV > 0) load(B);
+    const float* xrow = xs + g * XS;
+    float bv = 0.0f;
+    int bi = 0;
+    float a0 = 0.0f, a1 = 0.0f;
+    auto compute = [&](const KqBuf<TYPE, U>& b, int s0) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (s0 + u < nsb) {
+                float xv[16];
+                kq_x(xrow, s0 + u, xv);
+                kq_chunk<TYPE>(b.nb[u], b.hb[u], b.h[u], b.dm[u], g, xv, a0, a1);
+            }
+        }
+    };
+    const int nb = (nsb + U - 1) / U;  // buffers per row group
+    bool cur_b = false;                // whether the next buffer to compute is B
+    for (int rg = wid; rg < W.groups; rg += TW) {
+        const int lr = rg * 4 + r, row = row0 + lr;
+        const bool own = g == 0 && lr < W.rows;
+        const MvPre pre = mv_preload<EPI>(row, own, r, a, out);
+        a0 = a1 = 0.0f;
+        int i = 0;
+        if (cur_b) {  // (an odd number of buffers per row group: they swap)
+            compute(B, 0);
+            load(B);
+            i = 1;
+        }
+        for (; i + 1 < nb; i += 2) {
+            compute(A, i * U);
+            load(A);
+            compute(B, (i + 1) * U);
+            load(B);
+        }
+        if (i < nb) {
+            compute(A, i * U);
+            load(A);
+        }
+        cur_b = cur_b != ((nb & 1) != 0);
+        mv_epilogue<EPI>(kq_tree(a0, a1), row, own, r, row0 + W.rows, a, out, bv, bi, &pre);
+    }
+}
+
+// The decode matvec.  What bounds it: at 1024 row groups (one wave per SIMD) the latency of
+// the weight stream, so U is 8 chunks a buffer there (16 in flight per wave) and 4 otherwise;
+// past that the dequantisation (about 90 VALU instructions per 256 weights of 4 rows).  The
+// vector used to be staged by a loop of dependent 4-byte loads before the first weight load.
+template <int EPI, int NV, int U>
+__global__ __launch_bounds__(256, U == 4 && NV <= 4 ? 4 : 2) void matvec_kq_kernel(KqMats M, const float* __restrict__ x,
+                                                        const float* __restrict__ nw, float* __restrict__ out,
+                                                        MvArgs a) {
+    extern __shared__ __align__(16) float xs[];  // [16][XS]: lane pair g, 16 floats per chunk
+    __shared__ float red[18];
+    const int b = blockIdx.x;
+    const int i = b >= M.wg0[2] ? 2 : b >= M.wg0[1] ? 1 : 0;
+    const int wg = b - M.wg0[i], nwg = M.wg0[i + 1] - M.wg0[i];
+    switch (M.W[i].type) {  // (uniform over the workgroup)
+        case JY_Q4_K: kq_body<JY_Q4_K, EPI, NV, U>(M.W[i], wg, nwg, M.row0[i], x, nw, out, a, xs, red); break;
+        case JY_Q5_K: kq_body<JY_Q5_K, EPI, NV, U>(M.W[i], wg, nwg, M.row0[i], x, nw, out, a, xs, red); break;
+        default: kq_body<JY_Q6_K, EPI, NV, U>(M.W[i], wg, nwg, M.row0[i], x, nw, out, a, xs, red); break;
+    }
+}
+
+// gate and up of one type together: RMSNorm, both dots over the same staged vector (each
+// chunk's x read from LDS once for the two), out[j] = silu(gate_j) * up_j
+template <int TYPE, int NV>
+__global__ __launch_bounds__(256, NV <= 4 ? 4 : 2) void matvec_kq_pair_kernel(KQDev W0, KQDev W1, const float* __restrict__ x,
+                                                             const float* __restrict__ nw, float* __restrict__ out) {
+    extern __shared__ __align__(16) float xs[];
+    __shared__ float red[18];
+    constexpr int U = 2;
+    const int lane = threadIdx.x & 63, r = lane >> 4, g = lane & 15;
+    const int wid = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), TW = gridDim.x * 4;
+    const int nsb = W0.nsb, XS = 16 * nsb + 4, groups = W0.groups;
+    KqBuf<TYPE, U> A0, A1, B0, B1;
+    int lrg = min(wid, groups - 1), lp = 0;
+    auto load = [&](KqBuf<TYPE, U>& p, KqBuf<TYPE, U>& q) {
+        p.load(W0, lrg, lp, lane, r);
+        q.load(W1, lrg, lp, lane, r);
+        lp += U;
+        if (lp >= nsb) {
+            lp = 0;
+            lrg = min(lrg + TW, groups - 1);
+        }
+    };
+    kq_stage<NV, 4>(x, nw, W0.cols, XS, xs, red, [&]() { load(A0, A1); });
+    load(B0, B1);
+    const float* xrow = xs + g * XS;
+    float a0, a1, c0, c1;
+    auto compute = [&](const KqBuf<TYPE, U>& p, const KqBuf<TYPE, U>& q, int s0) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (s0 + u < nsb) {
+                float xv[16];
+                kq_x(xrow, s0 + u, xv);
+                kq_chunk<TYPE>(p.nb[u], p.hb[u], p.h[u], p.dm[u], g, xv, a0, a1);
+                kq_chunk<TYPE>(q.nb[u], q.hb[u], q.h[u], q.dm[u], g, xv, c0, c1);
+            }
+        }
+    };
+    const int nb = (nsb + U - 1) / U;
+    bool cur_b = false;
+    for (int rg = wid; rg < groups; rg += TW) {
+        a0 = a1 = c0 = c1 = 0.0f;
+        int i = 0;
+        if (cur_b) {
+            compute(B0, B1, 0);
+            load(B0, B1);
+            i = 1;
+        }
+        for (; i + 1 < nb; i += 2) {
+            compute(A0, A1, i * U);
+            load(A0, A1);
+            compute(B0, B1, (i + 1) * U);
+            load(B0, B1);
+        }
+        if (i < nb) {
+            compute(A0, A1, i * U);
+            load(A0, A1);
+        }
+        cur_b = cur_b != ((nb & 1) != 0);
+        const float yg = kq_tree(a0, a1), yu = kq_tree(c0, c1);
+        const int row = rg * 4 + r;
+        if (g == 0 && row < W0.rows) out[row] = silu_at(yg, row, W0.rows) * yu;
     }
 }
 
 size_t mv_kq_lds_bytes(int cols) { return (size_t)16 * (16 * (cols / 256) + 4) * sizeof(float); }
 
+static int g_kq_cus = 256;
+
+// workgroups of a matrix's launch: one row group per wave up to 4 workgroups per CU, past
+// that every workgroup the same number of row groups per wave (the vector is staged and
+// normalised once per workgroup)
+static int kq_wgs(const KQDev& W) {
+    const int max_waves = 16 * g_kq_cus, per = (W.groups + max_waves - 1) / max_waves;
+    return (W.groups + 4 * per - 1) / (4 * per);
+}
+
+static KqMats kq_mats(const KQDev* const* W, int n) {
+    KqMats M;
+    int wg = 0, row = 0;
+    for (int i = 0; i < 3; i++) {
+        M.W[i] = *W[i < n ? i : 0];
+        M.wg0[i] = wg;
+        M.row0[i] = row;
+        if (i < n) {
+            wg += kq_wgs(M.W[i]);
+            row += M.W[i].rows;
+        }
+    }
+    M.wg0[3] = wg;
+    // (matrices past n have no workgroups: their wg0 is the total)
+    return M;
+}
+
+template <int EPI, int NV>
+static void mv_kq(const KqMats& M, const float* x, const float* nw, float* out, const MvArgs& a, hipStream_t st) {
+    const dim3 grid((unsigned)M.wg0[3]), block(256);
+    const size_t lds = mv_kq_lds_bytes(M.W[0].cols);
+    if (M.wg0[3] <= g_kq_cus)
+        hipLaunchKernelGGL((matvec_kq_kernel<EPI, NV, 8>), grid, block, lds, st, M, x, nw, out, a);
+    else
+        hipLaunchKernelGGL((matvec_kq_kernel<EPI, NV, 4>), grid, block, lds, st, M, x, nw, out, a);
+}
+
+static bool is_kq(const DevW& w) { return w.type == JY_Q4_K || w.type == JY_Q5_K || w.type == JY_Q6_K; }
+
+static void mv_kq1(const DevW& W, const float* x, const float* nw, float* out, Epi epi, const float* aux,
+                   hipStream_t st) {
+    const KQDev* w[1] = {&W.kq};
+    const KqMats M = kq_mats(w, 1);
+    MvArgs a;
+    a.aux = aux;
+    if (nw) {
+        if (W.in <= KQ_NORM_MAX / 2)
+            mv_kq<EPI_STORE, 4>(M, x, nw, out, a, st);
+        else
+            mv_kq<EPI_STORE, 8>(M, x, nw, out, a, st);
+        return;
+    }
+    if (epi == EPI_STORE) mv_kq<EPI_STORE, 0>(M, x, nullptr, out, a, st);
+    if (epi == EPI_BIAS) mv_kq<EPI_BIAS, 0>(M, x, nullptr, out, a, st);
+    if (epi == EPI_RESID) mv_kq<EPI_RESID, 0>(M, x, nullptr, out, a, st);
+}
+
+bool launch_mv_norm(const DevW& W, const float* x, const float* nw, float* out, hipStream_t st) {
+    if (!is_kq(W) || W.in > KQ_NORM_MAX) return false;
+    mv_kq1(W, x, nw, out, EPI_STORE, nullptr, st);
+    return true;
+}
+
+bool launch_mv_qkv(const DevW* W, const float* x, const float* nw, float* qkv, const MvArgs& a, hipStream_t st) {
+    if (!is_kq(W[0]) || !is_kq(W[1]) || !is_kq(W[2]) || W[0].in > KQ_NORM_MAX) return false;
+    const KQDev* w[3] = {&W[0].kq, &W[1].kq, &W[2].kq};
+    if (W[0].in <= KQ_NORM_MAX / 2)
+        mv_kq<EPI_ROPE, 4>(kq_mats(w, 3), x, nw, qkv, a, st);
+    else
+        mv_kq<EPI_ROPE, 8>(kq_mats(w, 3), x, nw, qkv, a, st);
+    return true;
+}
+
 template <int TYPE>
-static void mv_kq(const KQDev& W, const float* x, float* out, Epi epi, const float* aux, hipStream_t st) {
-    const dim3 grid((unsigned)((W.groups + 3) / 4)), block(256);
-    const size_t lds = mv_kq_lds_bytes(W.cols);
-    if (epi == EPI_STORE) hipLaunchKernelGGL((matvec_kq_kernel<TYPE, EPI_STORE>), grid, block, lds, st, W, x, out, aux);
-    if (epi == EPI_BIAS) hipLaunchKernelGGL((matvec_kq_kernel<TYPE, EPI_BIAS>), grid, block, lds, st, W, x, out, aux);
-    if (epi == EPI_RESID) hipLaunchKernelGGL((matvec_kq_kernel<TYPE, EPI_RESID>), grid, block, lds, st, W, x, out, aux);
+static void mv_kq_pair(const KQDev& gate, const KQDev& up, const float* x, const float* nw, float* h, hipStream_t st) {
+    const dim3 grid((unsigned)kq_wgs(gate)), block(256);
+    const size_t lds = mv_kq_lds_bytes(gate.cols);
+    if (gate.cols <= KQ_NORM_MAX / 2)
+        hipLaunchKernelGGL((matvec_kq_pair_kernel<TYPE, 4>), grid, block, lds, st, gate, up, x, nw, h);
+    else
+        hipLaunchKernelGGL((matvec_kq_pair_kernel<TYPE, 8>), grid, block, lds, st, gate, up, x, nw, h);
+}
+
+bool launch_mv_gate_up(const DevW& gate, const DevW& up, const float* x, const float* nw, float* h, hipStream_t st) {
+    if (!is_kq(gate) || gate.type != up.type || gate.in > KQ_NORM_MAX) return false;
+    switch (gate.type) {
+        case JY_Q4_K: mv_kq_pair<JY_Q4_K>(gate.kq, up.kq, x, nw, h, st); break;
+        case JY_Q5_K: mv_kq_pair<JY_Q5_K>(gate.kq, up.kq, x, nw, h, st); break;
+        default: mv_kq_pair<JY_Q6_K>(gate.kq, up.kq, x, nw, h, st); break;
+    }
+    return true;
 }
 
 void launch_mv(const DevW& W, const float* x, float* out, Epi epi, const float* aux, hipStream_t st) {
@@ -263,27 +537,37 @@ void launch_mv(const DevW& W, const float* x, float* out, Epi epi, const float* 
             launch_matvec_q8(W.q8, x, nullptr, out, epi, a, st);
             break;
         }
-        case JY_Q4_K: mv_kq<JY_Q4_K>(W.kq, x, out, epi, aux, st); break;
-        case JY_Q5_K: mv_kq<JY_Q5_K>(W.kq, x, out, epi, aux, st); break;
-        case JY_Q6_K: mv_kq<JY_Q6_K>(W.kq, x, out, epi, aux, st); break;
-        default: break;
+        default: mv_kq1(W, x, nullptr, out, epi, aux, st); break;
     }
 }
 
-template <int TYPE>
-static hipError_t kq_attr() {
-    hipError_t e = hipSuccess;
-    for (const void* f : {reinterpret_cast<const void*>(&matvec_kq_kernel<TYPE, EPI_STORE>),
-                          reinterpret_cast<const void*>(&matvec_kq_kernel<TYPE, EPI_BIAS>),
-                          reinterpret_cast<const void*>(&matvec_kq_kernel<TYPE, EPI_RESID>)})
+hipError_t quant_init() {
+    int dev = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e == hipSuccess && cus > 0) g_kq_cus = cus;
+    for (const void* f : {reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, 0, 4>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, 0, 8>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, 4, 4>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, 4, 8>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, 8, 4>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, 8, 8>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_BIAS, 0, 4>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_BIAS, 0, 8>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_RESID, 0, 4>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_RESID, 0, 8>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_ROPE, 4, 4>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_ROPE, 4, 8>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_ROPE, 8, 4>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_ROPE, 8, 8>),
+                          reinterpret_cast<const void*>(&matvec_kq_pair_kernel<JY_Q4_K, 4>),
+                          reinterpret_cast<const void*>(&matvec_kq_pair_kernel<JY_Q4_K, 8>),
+                          reinterpret_cast<const void*>(&matvec_kq_pair_kernel<JY_Q5_K, 4>),
+                          reinterpret_cast<const void*>(&matvec_kq_pair_kernel<JY_Q5_K, 8>),
+                          reinterpret_cast<const void*>(&matvec_kq_pair_kernel<JY_Q6_K, 4>),
+                          reinterpret_cast<const void*>(&matvec_kq_pair_kernel<JY_Q6_K, 8>)})
         if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 2048);
     return e;
-}
-
-hipError_t quant_init() {
-    for (hipError_t e : {kq_attr<JY_Q4_K>(), kq_attr<JY_Q5_K>(), kq_attr<JY_Q6_K>()})
-        if (e != hipSuccess) return e;
-    return hipSuccess;
 }
 
 }  // namespace jy

@@ -865,24 +865,42 @@ void run_decode_layers(jyhip_model* m, Workspace& w, const KVDev& kv, const int*
             q8_matvec(m, D.gu, w.X, D.rms2, w.h, EPI_SWIGLU, none, st);
             q8_matvec(m, D.down, w.h, nullptr, w.X, EPI_RESID, none, st);
         } else if (m->wtype == WT_MIXED) {
+            // k-quant groups (q/k/v; gate/up of one type) in one launch with their RMSNorm; else
             // one kernel per matrix, each in its own type's order
             const int qd = m->qd, kvd = m->kvd;
-            const Epi qe = D.bqkv ? EPI_BIAS : EPI_STORE;
-            launch_rmsnorm(w.X, w.xn, D.rms1, H, 1, st);
-            launch_mv(D.w[0], w.xn, w.qkv, qe, D.bqkv, st);
-            launch_mv(D.w[1], w.xn, w.qkv + qd, qe, D.bqkv ? D.bqkv + qd : nullptr, st);
-            launch_mv(D.w[2], w.xn, w.qkv + qd + kvd, qe, D.bqkv ? D.bqkv + qd + kvd : nullptr, st);
-            launch_rope_pack(w.qkv, 1, pos0, state, m->nh, m->nkv, m->hd, m->cos_t, m->sin_t, kv, l, w.q8, w.qsc, st);
-            at.fused = false;
-            at.q8 = w.q8;
-            at.qsc = w.qsc;
-            at.row0 = 0;
+            MvArgs qa;
+            qa.aux = D.bqkv;
+            qa.state = state;
+            qa.pos0 = pos0;
+            qa.cos_t = m->cos_t;
+            qa.sin_t = m->sin_t;
+            qa.nh = m->nh;
+            qa.nkv = m->nkv;
+            qa.hd = m->hd;
+            if (launch_mv_qkv(D.w, w.X, D.rms1, w.qkv, qa, st)) {
+                at.fused = true;
+                at.qkv = w.qkv;
+            } else {
+                const Epi qe = D.bqkv ? EPI_BIAS : EPI_STORE;
+                launch_rmsnorm(w.X, w.xn, D.rms1, H, 1, st);
+                launch_mv(D.w[0], w.xn, w.qkv, qe, D.bqkv, st);
+                launch_mv(D.w[1], w.xn, w.qkv + qd, qe, D.bqkv ? D.bqkv + qd : nullptr, st);
+                launch_mv(D.w[2], w.xn, w.qkv + qd + kvd, qe, D.bqkv ? D.bqkv + qd + kvd : nullptr, st);
+                launch_rope_pack(w.qkv, 1, pos0, state, m->nh, m->nkv, m->hd, m->cos_t, m->sin_t, kv, l, w.q8, w.qsc,
+                                 st);
+                at.fused = false;
+                at.q8 = w.q8;
+                at.qsc = w.qsc;
+                at.row0 = 0;
+            }
             launch_attention(at, st);
             launch_mv(D.w[3], w.att, w.X, EPI_RESID, nullptr, st);
-            launch_rmsnorm(w.X, w.xn, D.rms2, H, 1, st);
-            launch_mv(D.w[4], w.xn, w.g, EPI_STORE, nullptr, st);
-            launch_mv(D.w[6], w.xn, w.u, EPI_STORE, nullptr, st);
-            launch_silu_mul(w.g, w.u, 0, 1, F, w.h, st);
+            if (!launch_mv_gate_up(D.w[4], D.w[6], w.X, D.rms2, w.h, st)) {
+                launch_rmsnorm(w.X, w.xn, D.rms2, H, 1, st);
+                launch_mv(D.w[4], w.xn, w.g, EPI_STORE, nullptr, st);
+                launch_mv(D.w[6], w.xn, w.u, EPI_STORE, nullptr, st);
+                launch_silu_mul(w.g, w.u, 0, 1, F, w.h, st);
+            }
             launch_mv(D.w[5], w.h, w.X, EPI_RESID, nullptr, st);
         } else {
             launch_rmsnorm(w.X, w.xn, D.rms1, H, 1, st);
@@ -1069,6 +1087,7 @@ void final_and_head(jyhip_model* m, Workspace& w, const float* xlast, bool argma
         }
         q8_matvec(m, m->lm_q8, xlast, m->final_rms, m->logits, argmax ? EPI_ARGMAX : EPI_STORE, a, m->stream);
     } else if (m->wtype == WT_MIXED) {
+        if (launch_mv_norm(m->lm_w, xlast, m->final_rms, m->logits, m->stream)) return;
         launch_rmsnorm(xlast, w.xn, m->final_rms, m->H, 1, m->stream);
         launch_mv(m->lm_w, w.xn, m->logits, EPI_STORE, nullptr, m->stream);
     } else {

@@ -70,3 +70,48 @@ def test_rmsnorm_widths(jy, oracle_lib, hidden):
     spec = dict(hidden=hidden, heads=1, kv=1, hd=16, inter=8, vocab=16, theta=10000.0, bias=False,
                 layers=[{s: QM.JY_F32 for s in QM.SLOTS}], embed=QM.JY_F32, lm=QM.JY_F32, tied=False)
     check_forward(jy, oracle_lib, spec, (3, 1))
+
+
+# k-quant decode: the launches with RMSNorm (q/k/v of different types, gate/up of one type) at
+# input widths under, at and over one register buffer of super-blocks (an odd number of buffers
+# per row: 256, 1280, 2304; the register norm's limits 4096 and 8192, and past it), row counts
+# that leave partial row groups and workgroups, more row groups than one pass of waves covers
+# (the lm_head), and groups whose types do not fuse
+@pytest.mark.parametrize("hidden,inter,types,vocab,bias", [
+    (256, 512, "445", 70, True), (1280, 256, "654", 1031, False), (2304, 768, "446", 66000, True),
+    (4096, 1024, "446", 300, False), (4352, 512, "556", 90, True), (8192, 256, "444", 41, False),
+    (8448, 256, "646", 41, False)])
+def test_kquant_decode_widths(jy, oracle_lib, hidden, inter, types, vocab, bias):
+    t = {"4": QM.JY_Q4_K, "5": QM.JY_Q5_K, "6": QM.JY_Q6_K}
+    q, k, v = (t[c] for c in types)
+    up = q if inter != 768 else k  # gate and up of different types once
+    layer = dict(Wq=q, Wk=k, Wv=v, Wo=k, W1=q, W2=v, W3=up)
+    spec = dict(hidden=hidden, heads=4, kv=2, hd=64, inter=inter, vocab=vocab, theta=10000.0, bias=bias,
+                layers=[layer], embed=v, lm=q, tied=False)
+    check_forward(jy, oracle_lib, spec, (2, 1, 1))
+    # the head: norm + lm_head in one launch, greedy picks against the oracle's logits
+    QM.SPECS["edge"] = spec
+    try:
+        m = QM.build_model("edge", 3)
+    finally:
+        del QM.SPECS["edge"]
+    d, keep = QM.desc_of(m)
+    cos, sin = rope_tables(oracle_lib, 16, 64, d.rope_theta)
+    prompt = QM.prompt_of(m, 3)
+    want, wl = np.zeros(17, np.int32), np.zeros(vocab, np.float32)
+    n = oracle_lib.jyo_generate(C.byref(d), ptr(prompt), 3, None, 0, ptr(cos), ptr(sin), 16, 4, 0.0, 1.0, ptr(want),
+                                None, ptr(wl))
+    g = jy.GpuModel(d, 16)
+    ids, _, logits = g.generate(prompt, 4, want_logits=True)
+    g.close()
+    assert ids.tolist() == want[:n].tolist()
+    assert bits_equal(logits, wl)
+
+
+# a q/k/v group with one matrix of another kind, and a gate/up pair of two types: one kernel each
+@pytest.mark.parametrize("wv,w3", [(QM.JY_Q8_0, QM.JY_Q4_K), (QM.JY_Q6_K, QM.JY_F16)])
+def test_kquant_groups_that_do_not_fuse(jy, oracle_lib, wv, w3):
+    layer = dict(Wq=QM.JY_Q4_K, Wk=QM.JY_Q4_K, Wv=wv, Wo=QM.JY_Q4_K, W1=QM.JY_Q4_K, W2=QM.JY_Q6_K, W3=w3)
+    spec = dict(hidden=512, heads=4, kv=2, hd=64, inter=768, vocab=64, theta=10000.0, bias=True, layers=[layer] * 2,
+                embed=QM.JY_Q6_K, lm=QM.JY_Q4_K, tied=False)
+    check_forward(jy, oracle_lib, spec, (1, 1, 2, 1))
