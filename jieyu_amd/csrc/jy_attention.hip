@@ -1257,6 +1257,7 @@ hipError_t matvec_split_init();
 hipError_t persist_init();
 hipError_t quant_init();
 hipError_t dense_init();
+hipError_t gemm_exact_init();
 
 hipError_t kernels_init() {
     int dev = 0, mx = 0;
@@ -1272,6 +1273,7 @@ hipError_t kernels_init() {
     if (e != hipSuccess) return e;
     e = quant_init();
     if (e == hipSuccess) e = dense_init();
+    if (e == hipSuccess) e = gemm_exact_init();
     if (e == hipSuccess) e = matvec_split_init();
     if (e == hipSuccess) e = persist_init();
     if (e == hipSuccess) e = gemm_mfma_init();

@@ -415,189 +415,6 @@ hipError_t dense_init() {
     return a != hipSuccess ? a : b;
 }
 
-// ---------------------------------------------------------------- prefill GEMMs (m > 1)
-
-// 64 tokens x 64 output rows per workgroup, 4x4 outputs per thread, k in order.
-// Quantized weights: acc = acc + x*w, rounded separately (the generic path of
-// matmul_q, libs/matmul_libs/matmul_q.h:145-161); the weight accessor dequantizes
-// exactly as dequant_block does.
-struct Q8Acc {
-    Q8Dev W;
-    __device__ float operator()(int R, int k) const { return q8_elem(W, R, k); }
-};
-struct KQAcc {
-    KQDev W;
-    __device__ float operator()(int R, int k) const { return kq_elem(W, R, k); }
-};
-
-template <class Acc, int EPI>
-__global__ __launch_bounds__(256) void gemm_quant_kernel(Acc W, int K, int N, int m, const float* __restrict__ A,
-                                                         float* __restrict__ Cm, int ldc,
-                                                         const float* __restrict__ aux) {
-    __shared__ float xs[32][68];
-    __shared__ float ws[32][68];
-    const int t = threadIdx.x, ti = t & 15, tj = t >> 4;
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    float acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = 0.0f;
-    const int lt = t >> 2, lc = (t & 3) * 8;  // loader: token/row lt, k offset lc
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        {
-            const int tok = m0 + lt;
-#pragma unroll
-            for (int c = 0; c < 8; c++) xs[lc + c][lt] = tok < m ? A[(size_t)tok * K + k0 + lc + c] : 0.0f;
-            const int R = n0 + lt;
-#pragma unroll
-            for (int c = 0; c < 8; c++) ws[lc + c][lt] = R < N ? W(R, k0 + lc + c) : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll 4
-        for (int kk = 0; kk < 32; kk++) {
-            const float4 xv = *reinterpret_cast<const float4*>(&xs[kk][ti * 4]);
-            const float4 wv = *reinterpret_cast<const float4*>(&ws[kk][tj * 4]);
-            const float xa[4] = {xv.x, xv.y, xv.z, xv.w}, wa[4] = {wv.x, wv.y, wv.z, wv.w};
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int b = 0; b < 4; b++) acc[a][b] = __fadd_rn(acc[a][b], __fmul_rn(xa[a], wa[b]));
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int a = 0; a < 4; a++) {
-        const int i = m0 + ti * 4 + a;
-        if (i >= m) continue;
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const int j = n0 + tj * 4 + b;
-            if (j >= N) continue;
-            float* c = Cm + (size_t)i * ldc + j;
-            if (EPI == EPI_STORE) *c = acc[a][b];
-            if (EPI == EPI_BIAS) *c = acc[a][b] + aux[j];
-            if (EPI == EPI_RESID) *c = *c + acc[a][b];
-        }
-    }
-}
-
-// dense [K][N] in the panel layout (f32, or f16 converted exactly): C = fma(A[i][p],
-// B[p][j], C) in order of p.
-template <typename T, int EPI>
-__global__ __launch_bounds__(256) void gemm_dense_kernel(const T* __restrict__ B, int K, int N, int m,
-                                                         const float* __restrict__ A, float* __restrict__ Cm, int ldc,
-                                                         const float* __restrict__ aux) {
-    __shared__ float xs[32][68];
-    __shared__ float ws[32][68];
-    const int t = threadIdx.x, ti = t & 15, tj = t >> 4;
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    float acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = 0.0f;
-    const int lt = t >> 2, lc = (t & 3) * 8;
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        const int tok = m0 + lt;
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const int k = k0 + lc + c;
-            xs[lc + c][lt] = (tok < m && k < K) ? A[(size_t)tok * K + k] : 0.0f;
-        }
-        // B rows k0..k0+31, columns n0..n0+63 of panel blockIdx.x: (32 / PER) x 64
-        // 16-byte pieces, piece pc = row piece pc / 64 of column pc % 64 (zeros past K
-        // come from the panel's padding; pieces past it are not read)
-        {
-            constexpr int PER = 16 / (int)sizeof(T), NPC = 32 / PER * 64 / 256;
-            const int nkb = (K + PER - 1) / PER;
-            const uint4* Pn = reinterpret_cast<const uint4*>(B) + (size_t)blockIdx.x * nkb * 64;
-#pragma unroll
-            for (int i = 0; i < NPC; i++) {
-                const int pc = t + 256 * i, kb = k0 / PER + pc / 64, col = pc % 64;
-                T el[PER];
-                if (kb < nkb) {
-                    dn_unpack<T>(Pn[(size_t)kb * 64 + col], el);
-                } else {
-#pragma unroll
-                    for (int u = 0; u < PER; u++) el[u] = (T)0;
-                }
-#pragma unroll
-                for (int u = 0; u < PER; u++) ws[(pc / 64) * PER + u][col] = dense_w(el, u);
-            }
-        }
-        __syncthreads();
-        const int kmax = K - k0 < 32 ? K - k0 : 32;
-        for (int kk = 0; kk < kmax; kk++) {
-            const float4 xv = *reinterpret_cast<const float4*>(&xs[kk][ti * 4]);
-            const float4 wv = *reinterpret_cast<const float4*>(&ws[kk][tj * 4]);
-            const float xa[4] = {xv.x, xv.y, xv.z, xv.w}, wa[4] = {wv.x, wv.y, wv.z, wv.w};
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int b = 0; b < 4; b++) acc[a][b] = __builtin_fmaf(xa[a], wa[b], acc[a][b]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int a = 0; a < 4; a++) {
-        const int i = m0 + ti * 4 + a;
-        if (i >= m) continue;
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const int j = n0 + tj * 4 + b;
-            if (j >= N) continue;
-            float* c = Cm + (size_t)i * ldc + j;
-            if (EPI == EPI_STORE) *c = acc[a][b];
-            if (EPI == EPI_BIAS) *c = acc[a][b] + aux[j];
-            if (EPI == EPI_RESID) *c = *c + acc[a][b];
-        }
-    }
-}
-
-template <class Acc>
-static void gemm_quant(const Acc& W, int K, int N, int m, const float* A, float* C, int ldc, const float* aux,
-                       Epi epi, hipStream_t st) {
-    const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((m + 63) / 64)), block(256);
-    if (epi == EPI_STORE)
-        hipLaunchKernelGGL((gemm_quant_kernel<Acc, EPI_STORE>), grid, block, 0, st, W, K, N, m, A, C, ldc, aux);
-    if (epi == EPI_BIAS)
-        hipLaunchKernelGGL((gemm_quant_kernel<Acc, EPI_BIAS>), grid, block, 0, st, W, K, N, m, A, C, ldc, aux);
-    if (epi == EPI_RESID)
-        hipLaunchKernelGGL((gemm_quant_kernel<Acc, EPI_RESID>), grid, block, 0, st, W, K, N, m, A, C, ldc, aux);
-}
-
-template <typename T>
-static void gemm_dense(const T* B, int K, int N, int m, const float* A, float* C, int ldc, const float* aux, Epi epi,
-                       hipStream_t st) {
-    const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((m + 63) / 64)), block(256);
-    if (epi == EPI_STORE)
-        hipLaunchKernelGGL((gemm_dense_kernel<T, EPI_STORE>), grid, block, 0, st, B, K, N, m, A, C, ldc, aux);
-    if (epi == EPI_BIAS)
-        hipLaunchKernelGGL((gemm_dense_kernel<T, EPI_BIAS>), grid, block, 0, st, B, K, N, m, A, C, ldc, aux);
-    if (epi == EPI_RESID)
-        hipLaunchKernelGGL((gemm_dense_kernel<T, EPI_RESID>), grid, block, 0, st, B, K, N, m, A, C, ldc, aux);
-}
-
-void launch_gemm_q8(const Q8Dev& W, int m, const float* A, float* C, const float* aux, Epi epi, hipStream_t st) {
-    gemm_quant(Q8Acc{W}, W.cols, W.rows, m, A, C, W.rows, aux, epi, st);
-}
-
-void launch_gemm_f32(const float* B, int K, int N, int m, const float* A, float* C, const float* aux, Epi epi,
-                     hipStream_t st) {
-    gemm_dense<float>(B, K, N, m, A, C, N, aux, epi, st);
-}
-
-void launch_gemm(const DevW& W, int m, const float* A, float* C, int ldc, const float* aux, Epi epi,
-                 hipStream_t st) {
-    switch (W.type) {
-        case JY_F32: gemm_dense(static_cast<const float*>(W.dense), W.in, W.out, m, A, C, ldc, aux, epi, st); break;
-        case JY_F16: gemm_dense(static_cast<const uint16_t*>(W.dense), W.in, W.out, m, A, C, ldc, aux, epi, st); break;
-        case JY_Q8_0: gemm_quant(Q8Acc{W.q8}, W.in, W.out, m, A, C, ldc, aux, epi, st); break;
-        default: gemm_quant(KQAcc{W.kq}, W.in, W.out, m, A, C, ldc, aux, epi, st); break;
-    }
-}
-
 __global__ void silu_mul_kernel(const float* __restrict__ g, const float* __restrict__ u, int interleaved, int m,
                                 int F, float* __restrict__ h) {
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;

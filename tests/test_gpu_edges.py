@@ -115,3 +115,25 @@ def test_kquant_groups_that_do_not_fuse(jy, oracle_lib, wv, w3):
     spec = dict(hidden=512, heads=4, kv=2, hd=64, inter=768, vocab=64, theta=10000.0, bias=True, layers=[layer] * 2,
                 embed=QM.JY_Q6_K, lm=QM.JY_Q4_K, tied=False)
     check_forward(jy, oracle_lib, spec, (1, 1, 2, 1))
+
+
+# the prompt GEMMs' tokens per wave (1, 2, 4, 8: by rows and columns), rows that leave a partial
+# wave and workgroup, 64-column tiles cut short, chunks of 256 cut to 32, 64, 96 and 224 (Q8_0),
+# dense widths under one piece, under one register buffer and with a tail
+@pytest.mark.parametrize("t,n,k", [
+    (QM.JY_Q8_0, 130, 32), (QM.JY_Q8_0, 65, 96), (QM.JY_Q8_0, 1, 320), (QM.JY_Q8_0, 4099, 480),
+    (QM.JY_Q4_K, 67, 256), (QM.JY_Q5_K, 4100, 512), (QM.JY_Q6_K, 129, 768),
+    (QM.JY_F32, 63, 3), (QM.JY_F32, 65, 66), (QM.JY_F32, 130, 513), (QM.JY_F32, 4099, 300),
+    (QM.JY_F16, 64, 7), (QM.JY_F16, 70, 130), (QM.JY_F16, 4098, 515)])
+@pytest.mark.parametrize("m", [2, 5, 17, 33, 70])
+def test_exact_gemm_tiles(jy, oracle_lib, t, n, k, m):
+    rng = np.random.default_rng(m + n + k + t)
+    w = QM.rand_matrix(rng, t, n, k)
+    wm = QM.WMat(w.ctypes.data_as(C.c_void_p), t)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    want = np.zeros((m, n), np.float32)
+    oracle_lib.jyo_matmul_w(C.byref(wm), m, n, k, ptr(a), ptr(want))
+    W = jy.WeightMatrix(w, t, n, k)
+    got = W.matmul(a)
+    W.close()
+    assert bits_equal(got, want)
