@@ -117,7 +117,7 @@ def test_kquant_groups_that_do_not_fuse(jy, oracle_lib, wv, w3):
     check_forward(jy, oracle_lib, spec, (1, 1, 2, 1))
 
 
-# the prompt GEMMs' tokens per wave (1, 2, 4, 8: by rows and columns), rows that leave a partial
+# the prompt GEMMs' tokens per wave (1, 2, 4, 8, 16: by rows and columns), rows that leave a partial
 # wave and workgroup, 64-column tiles cut short, chunks of 256 cut to 32, 64, 96 and 224 (Q8_0),
 # dense widths under one piece, under one register buffer and with a tail
 @pytest.mark.parametrize("t,n,k", [
@@ -127,6 +127,18 @@ def test_kquant_groups_that_do_not_fuse(jy, oracle_lib, wv, w3):
     (QM.JY_F16, 64, 7), (QM.JY_F16, 70, 130), (QM.JY_F16, 4098, 515)])
 @pytest.mark.parametrize("m", [2, 5, 17, 33, 70])
 def test_exact_gemm_tiles(jy, oracle_lib, t, n, k, m):
+    check_exact_gemm(jy, oracle_lib, t, n, k, m)
+
+
+# the widest form (16 tokens per wave): a partial last tile and wave, dense K under 16 and with a tail
+@pytest.mark.parametrize("t,n,k,m", [
+    (QM.JY_Q8_0, 24003, 96, 61), (QM.JY_Q6_K, 24003, 256, 50), (QM.JY_F32, 3100, 83, 200), (QM.JY_F32, 3100, 9, 200),
+    (QM.JY_F16, 24003, 83, 61), (QM.JY_F16, 3100, 150, 211)])
+def test_exact_gemm_wide_tiles(jy, oracle_lib, t, n, k, m):
+    check_exact_gemm(jy, oracle_lib, t, n, k, m)
+
+
+def check_exact_gemm(jy, oracle_lib, t, n, k, m):
     rng = np.random.default_rng(m + n + k + t)
     w = QM.rand_matrix(rng, t, n, k)
     wm = QM.WMat(w.ctypes.data_as(C.c_void_p), t)
