@@ -47,13 +47,6 @@ __device__ __forceinline__ void gemm_store(const float (&acc)[T], int i0, int m,
     }
 }
 
-// blocks in launch order go round the 8 XCDs: give each XCD a contiguous run of tiles, so
-// that the row groups of one column tile share its L2
-__device__ __forceinline__ int xcd_tile(int id, int total) {
-    const int x = id & 7, q = total >> 3, r = total & 7;
-    return x * q + min(x, r) + (id >> 3);
-}
-
 // ---------------------------------------------------------------- quantized weights
 
 // One workgroup: 64 weight rows, 4 waves of T tokens.  Per 256 weights of a row (a chunk of 8
@@ -243,7 +236,6 @@ __global__ __launch_bounds__(256) void gemm_exact_kernel(Dev W, int m, int mt, i
 // columns (one per lane of B) of one k per instruction, the matrix cores running beside the
 // vector unit, which is left with the add.  One register of A holds 64 / TT k of the TT
 // tokens (lane TT j + t: token t), of which the instruction's broadcast picks one (ABID j).
-typedef float f16_t __attribute__((ext_vector_type(16)));
 
 template <int TT> struct Outer;
 template <> struct Outer<16> {
@@ -271,7 +263,6 @@ __device__ __forceinline__ void static_for(F&& f) {
         static_for<I + 1, N>(f);
     }
 }
-__device__ __forceinline__ float f4_get(const float4& v, int e) { return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w; }
 
 // the epilogue of MT tiles of TT tokens x 64 columns
 template <int TT, int MT>

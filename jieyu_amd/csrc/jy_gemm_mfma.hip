@@ -12,17 +12,29 @@
 // the 2^-22 relative split of the activations.
 //
 // Layout.  The matrix is kept a second time for these kernels (built when the mode is
-// enabled): for every tile of 16 rows and every block, the 512 bytes the 64 lanes of an
-// MFMA's B operand read, lane l = c + 16 G (row c of the tile, k = 8G .. 8G+7 of the
-// block) holding 8 bytes; and the block scales as fp32, four blocks of a row together.
-// The A operand takes lane l = r + 16 G for row r and the same k = 8G .. 8G+7: whatever
-// order the instruction gives the four lane groups' k, A and B agree on it.
+// enabled): for every tile of 16 rows and every block 512 bytes, slot c + 16 g (row c of the
+// tile) holding the 16 bytes k = 16 g .. 16 g + 15 of the block, which one lane of the B
+// operand takes at once; and the block scales as fp32, four blocks of a row together (zero
+// past the last block).  v_mfma_f32_32x32x16_f16 takes 16 k from two lane groups of 8; the
+// kernel gives lane group g of the h-th of a block's two instructions k = 16 g + 8 h .. + 7
+// in both operands: whatever order the instruction gives them, A and B agree on it.
 //
-// Tiling.  A workgroup of 2 x 2 waves computes 64 rows (tokens) x 64 NT columns (matrix
-// rows), each wave 32 x 16 NT: 2 x NT tiles of 16 x 16, acc in the MFMA C layout (lane l
-// holds rows 4 (l/16) .. +3 of column l % 16).  The operands reach LDS by global -> LDS DMA
-// three blocks deep (activation parts in operand order, weights as stored, block scales),
-// one workgroup barrier per block; each wave converts its weight fragments to fp16.
+// Tiling.  A workgroup of 4 waves computes 32 MT rows (tokens) x 128 NT columns (matrix
+// rows), each wave all the rows of its 32 NT columns.  So a wave alone uses its weights and
+// takes them straight into registers (16 bytes per lane, reloaded for the next step as each
+// block is used up), and only the activations, which all four share, go through LDS, by
+// global -> LDS DMA, four blocks a step and two steps deep, with one barrier per step.
+//
+// What bounds it: at many rows, instruction issue and the vector memory path together; at few,
+// the latency of a wave's chain and the weights' bytes.  Measured on the way (gate/up of
+// Llama-3-8B, 28672 x 4096, 1024 rows):
+//   16x16x32 tiles, everything through LDS, a barrier per block      545-565 us
+//   the same with 32x32x16 tiles (16x16x32 takes 4 passes and leaves the vector unit no
+//   slot beside it; 32x32x16 takes 8 and hides ~5 ns of vector work) 554
+//   weights to registers, a barrier per 4 blocks                     559
+//   DMA by whole 128-byte lines and 16-byte weight loads             497
+// (the number of cache lines a load instruction touches was the limit: with the loads left out
+// the second form took 393 us, the matrix instructions alone 328, 1.47 PFLOP/s.)
 #include <algorithm>
 #include <cstddef>
 
@@ -31,14 +43,15 @@
 
 namespace jy {
 
-static constexpr int GM_TILE = 128;  // activation rows are padded to a multiple of this
+static constexpr int GM_TILE = 64;  // activation rows are padded to a multiple of this
+static constexpr int GM_KB = 4;     // 32-weight blocks per step of the GEMM
 
 typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------- the matrix copy
 
-// one thread per (16-row tile t, block b, lane l): the 8 weights of row 16t + (l % 16),
-// k = 32b + 8(l/16) .. +7, from the lane-pair layout (slot r*16 + g of chunk b/8 holds
+// one thread per (16-row tile t, block b, l): the 8 weights of row 16t + (l % 16),
+// k = 32b + 8(l/16) .. +7, into half (l/16) % 2 of slot (l % 16) + 16 (l/32), from the lane-pair layout (slot r*16 + g of chunk b/8 holds
 // weights 2g, 2g+1 of each of its 8 blocks at bytes 2j, 2j+1); the scales of blocks
 // 4*b4 .. 4*b4+3 of each row by the threads with l < 16 and b % 4 == 0
 __global__ void mfma_repack_kernel(Q8Dev W, Q8MfmaDev M) {
@@ -62,7 +75,7 @@ __global__ void mfma_repack_kernel(Q8Dev W, Q8MfmaDev M) {
         w0 = v[0] | (v[1] << 16);
         w1 = v[2] | (v[3] << 16);
     }
-    uint2* dst = reinterpret_cast<uint2*>(M.q + (tb * 64 + l) * 8);
+    uint2* dst = reinterpret_cast<uint2*>(M.q + tb * 512 + (((G >> 1) * 16 + (l % 16)) * 2 + (G & 1)) * 8);
     *dst = make_uint2(w0, w1);
     if (l < 16 && (b & 3) == 0) {
         float4 dv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -148,9 +161,9 @@ __global__ __launch_bounds__(256) void mfma_norm_split_kernel(const float* __res
 }
 
 // The same two kernels with the row in registers: NV float4s per thread (element
-// 4 (tid + 256 j) .. +3 in v[j]), one read of the row, 16-byte loads and 8-byte stores of
-// four halves; the same arithmetic element by element (K a multiple of 4, K <= 1024 NV).
-template <int NV>
+// 4 (tid + TH j) .. +3 in v[j], TH threads), one read of the row, 16-byte loads and 8-byte stores of
+// four halves; the same arithmetic element by element (K a multiple of 4, K <= 4 TH NV).
+template <int NV, int TH = 256>
 __device__ __forceinline__ void split_row4(const float4 (&v)[NV], int K, int row, _Float16* __restrict__ hi,
                                            _Float16* __restrict__ lo, float* __restrict__ unscale, float* red) {
     const int tid = threadIdx.x;
@@ -162,6 +175,8 @@ __device__ __forceinline__ void split_row4(const float4 (&v)[NV], int K, int row
     if ((tid & 63) == 0) red[tid >> 6] = amax;
     __syncthreads();
     amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+#pragma unroll
+    for (int w = 4; w < TH / 64; w++) amax = fmaxf(amax, red[w]);
     int ex = 0;
     if (amax > 0.0f) frexpf(amax, &ex);
     const int s = amax > 0.0f ? min(max(14 - ex, -100), 100) : 0;
@@ -171,7 +186,7 @@ __device__ __forceinline__ void split_row4(const float4 (&v)[NV], int K, int row
     _Float16* w = lo + (size_t)row * K;
 #pragma unroll
     for (int j = 0; j < NV; j++) {
-        const int k4 = tid + 256 * j;
+        const int k4 = tid + TH * j;
         if (4 * k4 >= K) break;
         const float e[4] = {v[j].x * up, v[j].y * up, v[j].z * up, v[j].w * up};
         h4_t vh, vl;
@@ -185,21 +200,21 @@ __device__ __forceinline__ void split_row4(const float4 (&v)[NV], int K, int row
     }
 }
 
-template <int NV>
-__global__ __launch_bounds__(256) void mfma_split4_kernel(const float* __restrict__ A, int m, int K,
+template <int NV, int TH = 256>
+__global__ __launch_bounds__(TH) void mfma_split4_kernel(const float* __restrict__ A, int m, int K,
                                                           _Float16* __restrict__ hi, _Float16* __restrict__ lo,
                                                           float* __restrict__ unscale) {
-    __shared__ float red[4];
+    __shared__ float red[TH / 64];
     const int row = blockIdx.x;
     const bool live = row < m;
     const float4* a4 = reinterpret_cast<const float4*>(A + (size_t)row * K);
     float4 v[NV];
 #pragma unroll
     for (int j = 0; j < NV; j++) {
-        const int k4 = threadIdx.x + 256 * j;
+        const int k4 = threadIdx.x + TH * j;
         v[j] = live && 4 * k4 < K ? a4[k4] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
-    split_row4<NV>(v, K, row, hi, lo, unscale, red);
+    split_row4<NV, TH>(v, K, row, hi, lo, unscale, red);
 }
 
 // (kz > 1: X's rows first take the residual add of a GEMM split over K whose sum was
@@ -267,8 +282,10 @@ __global__ __launch_bounds__(256) void mfma_norm_split4_kernel(float* __restrict
     split_row4<NV>(v, K, row, hi, lo, unscale, red);
 }
 
-// float4s per thread for a row of K (0: the scalar kernels: K not a multiple of 4 or past 16384)
-static int split_nv(int K) {
+// float4s per thread (of 256) for a row of K (0: the scalar kernels, K not a multiple of 4 or
+// past 16384; 32: 16 for each of 512 threads, up to 32768, where the caller has that form)
+static int split_nv(int K, bool wide = false) {
+    if (wide && K % 4 == 0 && K > 16384 && K <= 32768) return 32;
     if (K % 4 || K > 16384) return 0;
     const int n = (K + 1023) / 1024;
     return n <= 1 ? 1 : n <= 2 ? 2 : n <= 4 ? 4 : n <= 8 ? 8 : 16;
@@ -293,29 +310,21 @@ void launch_mfma_norm_split(float* X, int m, int mp, int K, const float* nw, _Fl
 
 void launch_mfma_split(const float* A, int m, int mp, int K, _Float16* hi, _Float16* lo, float* unscale,
                        hipStream_t st) {
-    switch (split_nv(K)) {
+    switch (split_nv(K, true)) {
         case 1: hipLaunchKernelGGL(mfma_split4_kernel<1>, dim3(mp), dim3(256), 0, st, A, m, K, hi, lo, unscale); break;
         case 2: hipLaunchKernelGGL(mfma_split4_kernel<2>, dim3(mp), dim3(256), 0, st, A, m, K, hi, lo, unscale); break;
         case 4: hipLaunchKernelGGL(mfma_split4_kernel<4>, dim3(mp), dim3(256), 0, st, A, m, K, hi, lo, unscale); break;
         case 8: hipLaunchKernelGGL(mfma_split4_kernel<8>, dim3(mp), dim3(256), 0, st, A, m, K, hi, lo, unscale); break;
         case 16: hipLaunchKernelGGL(mfma_split4_kernel<16>, dim3(mp), dim3(256), 0, st, A, m, K, hi, lo, unscale); break;
+        // (18944 wide, 61 rows: 33 us by the scalar kernel)
+        case 32: hipLaunchKernelGGL((mfma_split4_kernel<16, 512>), dim3(mp), dim3(512), 0, st, A, m, K, hi, lo, unscale); break;
         default: hipLaunchKernelGGL(mfma_split_kernel, dim3(mp), dim3(256), 0, st, A, m, K, hi, lo, unscale); break;
     }
 }
 
-// ---------------------------------------------------------------- the GEMM, staged by DMA
-//
-// Per block: the hi-part MFMA, the lo-part MFMA into the same sum, one fp32 fma with the
-// block scale.  The operands are brought to LDS by global -> LDS DMA, S blocks deep, with
-// a wave tile of
-// 16 MT token rows x 16 NT columns (a workgroup of 2 x 2 waves: 32 MT x 32 NT).  The
-// weights stay int8 in LDS (8 bytes per lane per 16 x 32 tile) and become fp16 per
-// fragment (q8_to_h8).  Per block a wave reads 2 MT KiB of activation fragments and NT / 2
-// KiB of weights from LDS for 2 MT NT matrix operations.  (A register-staged form with one
-// 32-weight block per barrier, 64 x 64 per wave and the weight fragments read twice was
-// bound by LDS reads: gate/up at 1024 tokens 682 us against 576 here.)
+// ---------------------------------------------------------------- the GEMM
 
-// global -> LDS DMA (16 or 4 bytes per lane: lane l writes at the M0 base + l * size),
+// global -> LDS DMA (16 bytes per lane: lane l writes at the M0 base + 16 l),
 // issued as inline assembly: the compiler cannot tell a DMA's LDS destination from the LDS
 // the waves read and would wait for every DMA before each LDS access; the kernel instead
 // waits for its own DMAs explicitly before the barrier that publishes a stage.  The asm sets
@@ -326,9 +335,6 @@ void launch_mfma_split(const float* A, int m, int mp, int K, _Float16* hi, _Floa
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma_b128(const void* g, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ void dma_b32(const void* g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
 }
 #pragma clang diagnostic pop
 __device__ __forceinline__ uint32_t lds_byte_addr(const void* p) {
@@ -342,252 +348,179 @@ __device__ __forceinline__ void wait_vm() {
     __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
 }
 
-// one stage: activation fragments [part][row tile][lane], weights [column tile][lane]
-// (8 bytes: lanes 0..31 of a 16-byte DMA cover one tile), block scales [column tile][row]
-template <int MT, int NT>
-struct G2Stage {
-    h8_t a[2][2 * MT][64];
-    uint2 b[2 * NT][64];
-    float d[2 * NT][16];
-};
-
-template <int EPI, int MT, int NT, int S>
-__global__ __launch_bounds__(256, 2) void gemm_q8_mfma2_kernel(Q8MfmaDev W, int m, int K, const _Float16* __restrict__ ahi,
-                                                            const _Float16* __restrict__ alo,
-                                                            const float* __restrict__ unscale, float* __restrict__ C,
-                                                            int ldc, const float* __restrict__ aux) {
-    static_assert(MT == 2 || MT == 4, "row tiles per wave");
-    static_assert(NT == 4 || NT == 8, "column tiles per wave");
-    static_assert(S == 3 || S == 4, "stages");
-    using St = G2Stage<MT, NT>;
-    extern __shared__ __align__(16) unsigned char g2smem[];
-    St* stg = reinterpret_cast<St*>(g2smem);
+template <int EPI, int MT, int NT>
+__global__ __launch_bounds__(256, 2) void gemm_q8_mfma_kernel(
+    Q8MfmaDev W, int m, int K, int mtiles, int total, int nbz, const _Float16* __restrict__ ahi,
+    const _Float16* __restrict__ alo, const float* __restrict__ unscale, float* __restrict__ C, int ldc,
+    const float* __restrict__ aux) {
+    constexpr int KB = GM_KB, NW = 4, R = 32 * MT, CC = 32 * NT * NW, RT = R / 16;
+    constexpr int NA = 2 * KB * RT / NW;  // DMA instructions per wave and step
+    extern __shared__ __align__(16) unsigned char gsmem[];
+    h8_t(*As)[2][RT][KB][64] = reinterpret_cast<h8_t(*)[2][RT][KB][64]>(gsmem);  // [buffer][part][row tile][block][lane]
+    constexpr uint32_t ABUF = 2u * RT * KB * 1024;
     const int tid = threadIdx.x, l = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave & 1, wn = wave >> 1;
-    const int c = l & 15, G = l >> 4;
-    const int rowt = blockIdx.x * 32 * MT;  // the workgroup's first token row
-    const int tilet = blockIdx.y * 2 * NT;  // its first 16-column tile
+    const int tile = xcd_tile(blockIdx.x, total);
+    const int ct = tile / mtiles;
+    const int rowt = (tile - ct * mtiles) * R;  // the workgroup's first token row
+    const int tilet = ct * (CC / 16) + wave * 2 * NT;  // the wave's first 16-column tile
     const int nb = W.nb;
-    // the workgroup's K slice: blocks [b0, b1) of gridDim.z slices of nbz (all of them with
-    // one slice), its sums into C's slice z ([z][m][ldc]: the partials a sum kernel adds)
-    const int nbz = (nb + (int)gridDim.z - 1) / (int)gridDim.z;
-    const int b0 = (int)blockIdx.z * nbz, b1 = min(nb, b0 + nbz);
-    C += (size_t)blockIdx.z * m * ldc;
-    const uint32_t base = __builtin_amdgcn_readfirstlane(lds_byte_addr(g2smem));
-    constexpr int PW = MT + NT / 4 + 1;  // DMA instructions per wave per block
+    // the workgroup's K slice: blocks [b0, b1), its sums into C's slice y ([z][m][ldc]: the
+    // partials a sum kernel adds); nbz is a multiple of KB
+    const int b0 = (int)blockIdx.y * nbz, b1 = min(nb, b0 + nbz);
+    C += (size_t)blockIdx.y * m * ldc;
+    const uint32_t base = __builtin_amdgcn_readfirstlane(lds_byte_addr(gsmem));
 
-    // block b into stage s: this wave's share of the 4 MT activation, NT weight and 4 scale
-    // DMA instructions (the same count for every wave)
-    auto issue = [&](int b, int s) {
-        const uint32_t sb = base + (uint32_t)(s * sizeof(St));
+    // One DMA instruction brings 8 rows x 128 bytes (two blocks): row l / 8, and of its eight
+    // 16-byte pieces the one of slot l % 8, slots being pieces exchanged by the row's low bits
+    // (piece = slot ^ row % 8), so that the fragment reads spread over the banks.
+    static_assert(KB == 4 && NA % 4 == 0, "whole 16-row tiles per wave: 8-row halves x block pairs");
+    const _Float16* asrc[NA / 4];
 #pragma unroll
-        for (int j = 0; j < MT; j++) {
-            const int i = wave * MT + j, part = i / (2 * MT), rt = i % (2 * MT);
-            const _Float16* src = (part ? alo : ahi) + (size_t)(rowt + 16 * rt + c) * K + 32 * b + 8 * G;
-            dma_b128(src, sb + (uint32_t)(offsetof(St, a) + (size_t)(part * 2 * MT + rt) * 64 * 16));
-        }
+    for (int j = 0; j < NA / 4; j++) {
+        const int i = wave * (NA / 4) + j, part = i / RT, rt = i % RT;
+        asrc[j] = (part ? alo : ahi) + (size_t)(rowt + 16 * rt + (l >> 3)) * K;
+    }
+    const int apc = 8 * ((l & 7) ^ (l >> 3));
+    auto issue_a = [&](int b, int buf) {
 #pragma unroll
-        for (int j = 0; j < NT / 4; j++) {
-            const int jj = wave * (NT / 4) + j, t = 2 * jj + (l >> 5);
-            const int tg = min(tilet + t, W.tiles - 1);
-            const int8_t* src = W.q + ((size_t)tg * nb + b) * 512 + (l & 31) * 16;
-            dma_b128(src, sb + (uint32_t)(offsetof(St, b) + (size_t)(2 * jj) * 512));
-        }
-        {
-            const int f = wave * 8 * NT + l, t = f >> 4, r = f & 15;
-            const int tg = min(tilet + t, W.tiles - 1);
-            const float* src = W.d + ((size_t)(tg * W.nb4 + (b >> 2)) * 16 + r) * 4 + (b & 3);
-            if (l < 8 * NT) dma_b32(src, sb + (uint32_t)(offsetof(St, d) + (size_t)wave * 8 * NT * 4));
-        }
+        for (int j = 0; j < NA / 4; j++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)  // i & 1: rows + 8; i >> 1: blocks + 2
+                dma_b128(asrc[j] + (size_t)(i & 1) * 8 * K + min(32 * (b + 2 * (i >> 1)) + apc, K - 8),
+                         base + buf * ABUF + (uint32_t)((wave * (NA / 4) + j) * 4 + 2 * (i >> 1) + (i & 1)) * 1024);
+    };
+    // this lane's column: tile (l & 31) / 16 of a pair, row l % 16 of it; its k: 16 (l / 32) .. +15
+    const int t0 = min(tilet, W.tiles - 1);
+    const __amdgpu_buffer_rsrc_t qr = __builtin_amdgcn_make_buffer_rsrc(
+        W.q + (size_t)t0 * nb * 512, 0, (int)min((size_t)(W.tiles - t0) * nb * 512, (size_t)0x7fffffff), 0x00020000);
+    const __amdgpu_buffer_rsrc_t dr = __builtin_amdgcn_make_buffer_rsrc(
+        W.d + (size_t)t0 * W.nb4 * 64, 0, (int)min((size_t)(W.tiles - t0) * W.nb4 * 256, (size_t)0x7fffffff), 0x00020000);
+    const int qo = ((l & 31) >> 4) * nb * 512 + (l & 15) * 16 + 256 * (l >> 5);
+    const int dof = ((l & 31) >> 4) * W.nb4 * 256 + (l & 15) * 16;
+    uint4 q[KB][NT];
+    float4 dcur[NT], dnxt[NT];
+    auto load_b = [&](int b, int kb) {
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+            q[kb][nt] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(qr, qo, (nt * 2 * nb + b + kb) * 512, 0));
+    };
+    auto load_d = [&](int b, float4(&d)[NT]) {
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) d[nt] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(dr, dof, (nt * 2 * W.nb4 + b / 4) * 256, 0));
     };
 
-    f4_t acc[MT][NT];
+    auto mm = [](h8_t a, h8_t b, f16_t c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); };
+    f16_t acc[MT][NT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++) acc[mt][nt] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-
-    // The narrow tile (NT = 4) runs the block loop software-pipelined; the wide tile's
-    // registers do not hold a second set of fragments well (238 VGPRs: gate/up 594 -> 628 us),
-    // so it reads each block's fragments after its barrier.
-    if constexpr (NT == 4) {
-        // Software-pipelined over blocks: while the matrix cores work on block b from registers,
-        // the fragments of block b + 1 are read from LDS into the other register set.  S blocks
-        // are in LDS or in flight: block b + S goes into block b's stage once every wave has
-        // read block b (the barrier before block b + 1's reads).
-        struct Frag {
-            h8_t ah[MT], al[MT];
-            uint2 q[NT];
-            float dj[NT];
-        };
-        auto read_frag = [&](int b, Frag& f) {
-            const St& T = stg[(b - b0) % S];
+        for (int nt = 0; nt < NT; nt++) acc[mt][nt] = f16_t(0.0f);
+    // fragment address: 16-row tile (l & 31) / 16, row l % 16 in it, piece 4 (kb % 2) + 2 (l / 32) + h
+    const int fr = ((l & 31) >> 4) * 4 * 64 + ((l >> 3) & 1) * 64 + (l & 7) * 8;
+    auto block = [&](int buf, int kb) {
+        h8_t ah[MT][2], al[MT][2];
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                f.ah[mt] = T.a[0][wm * MT + mt][l];
-                f.al[mt] = T.a[1][wm * MT + mt][l];
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int sl = fr + ((4 * (kb & 1) + 2 * (l >> 5) + h) ^ (l & 7)) + (kb >> 1) * 128;
+                ah[mt][h] = (&As[buf][0][mt * 2][0][0])[sl];
+                al[mt][h] = (&As[buf][1][mt * 2][0][0])[sl];
             }
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
-                f.q[nt] = T.b[wn * NT + nt][l];
-                f.dj[nt] = T.d[wn * NT + nt][c];
-            }
-        };
-        // the wait for block b's DMAs when `later` blocks were issued after it
-        auto wait_block = [&](int later) {
-            if (later >= S - 1)
-                wait_vm<(S - 1) * PW>();
-            else if (later == S - 2)
-                wait_vm<(S - 2) * PW>();
-            else if (S > 3 && later == 1)
-                wait_vm<(S > 3 ? PW : 0)>();
-            else
-                wait_vm<0>();
-        };
-        auto compute = [&](const Frag& f) {
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
-                const h8_t bq = q8_to_h8(f.q[nt].x, f.q[nt].y);
-                f4_t t[MT];
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-                    t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.ah[mt], bq, f4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++) t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.al[mt], bq, t[mt], 0, 0, 0);
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) acc[mt][nt][i] = __builtin_fmaf(f.dj[nt], t[mt][i], acc[mt][nt][i]);
-            }
-        };
-        // block b from cur; block b + 1 (if any) into nxt
-        auto step = [&](int b, const Frag& cur, Frag& nxt) {
-            if (b + 1 < b1) {
-                // issued after block b + 1 so far: blocks b + 2 .. min(b + S - 1, b1 - 1)
-                wait_block(min(S - 2, b1 - b - 2));
-                __syncthreads();  // block b + 1 is in LDS; every wave has read block b
-                if (b + S < b1) issue(b + S, (b - b0) % S);
-                read_frag(b + 1, nxt);
-            }
-            compute(cur);
-        };
-
-#pragma unroll
-        for (int s = 0; s < S; s++)
-            if (b0 + s < b1) issue(b0 + s, s);
-        Frag fa, fb;
-        if (b0 < b1) {
-            wait_block(min(S - 1, b1 - b0 - 1));
-            __syncthreads();
-            read_frag(b0, fa);
-        }
-        int b = b0;
-        for (; b + 1 < b1; b += 2) {
-            step(b, fa, fb);
-            step(b + 1, fb, fa);
-        }
-        if (b < b1) step(b, fa, fb);
-    } else {
-#pragma unroll
-        for (int s = 0; s < S - 1; s++)
-            if (b0 + s < b1) issue(b0 + s, s);
-        for (int b = b0; b < b1; b++) {
-            // block b has landed once at most the DMAs of the S - 2 blocks after it are pending
-            const int after = min(b1 - 1 - b, S - 2);
-            if (after >= S - 2)
-                wait_vm<(S - 2) * PW>();
-            else if (S > 3 && after == 1)
-                wait_vm<(S > 3 ? PW : 0)>();
-            else
-                wait_vm<0>();
-            __syncthreads();  // every wave's DMAs of block b are in LDS; block b - 1 is done
-            if (b + S - 1 < b1) issue(b + S - 1, (b - b0 + S - 1) % S);
-            const St& T = stg[(b - b0) % S];
-            h8_t ah[MT], al[MT];
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                ah[mt] = T.a[0][wm * MT + mt][l];
-                al[mt] = T.a[1][wm * MT + mt][l];
-            }
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
-                const uint2 q = T.b[wn * NT + nt][l];
-                const h8_t bq = q8_to_h8(q.x, q.y);
-                const float dj = T.d[wn * NT + nt][c];
-                f4_t t[MT];
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-                    t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[mt], bq, f4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++) t[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[mt], bq, t[mt], 0, 0, 0);
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) acc[mt][nt][i] = __builtin_fmaf(dj, t[mt][i], acc[mt][nt][i]);
-            }
-        }
-    }
-
-    // epilogue: acc[mt][nt][i] is C[row][col] before the row's unscale; the rows' factors
-    // are loaded together first, so no store waits for a load of its own
-    const int N = W.rows;
-    float us[MT][4];
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int row = rowt + wm * 16 * MT + 16 * mt + 4 * G + i;
-            us[mt][i] = row < m ? unscale[row] : 0.0f;
-        }
-    if (EPI == EPI_SWIGLU) {
-        // the gate/up matrix's rows 2j, 2j+1 are gate_j, up_j: columns 2j and 2j+1 of C lie in
-        // lanes c and c + 1 of a tile; the even lane writes h[row][j] = silu(gate) * up with
-        // the reference's SiLU of element row * F + j of the m x F array (silu_mul_kernel)
-        const int F = N >> 1;
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) {
-            if (tilet + wn * NT + nt >= W.tiles) continue;  // (uniform over the wave)
-            const int col = 16 * (tilet + wn * NT + nt) + c;
+            const h8_t bq[2] = {q8_to_h8(q[kb][nt].x, q[kb][nt].y), q8_to_h8(q[kb][nt].z, q[kb][nt].w)};
+            const float dv = f4_get(dcur[nt], kb);
+            f16_t t[MT];
+            // (high parts first: the low parts ahead of them would save no instruction, and the error
+            // against 64 bits would be 1-3 % larger)
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) t[mt] = mm(ah[mt][0], bq[0], f16_t(0.0f));
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) t[mt] = mm(ah[mt][1], bq[1], t[mt]);
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) t[mt] = mm(al[mt][0], bq[0], t[mt]);
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) t[mt] = mm(al[mt][1], bq[1], t[mt]);
 #pragma unroll
             for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int row = rowt + wm * 16 * MT + 16 * mt + 4 * G + i;
-                    const float y = acc[mt][nt][i] * us[mt][i];
+                for (int i = 0; i < 16; i++) acc[mt][nt][i] = __builtin_fmaf(dv, t[mt][i], acc[mt][nt][i]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // (a step past the last block: the scales there are zero, the activations repeated, the
+    // weights another tile's or, past the matrix, zero)
+    if (b0 < b1) {
+        issue_a(b0, 0);
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++) load_b(b0, kb);
+        load_d(b0, dcur);
+        int buf = 0;
+        for (int b = b0; b < b1; b += KB, buf ^= 1) {
+            wait_vm<0>();
+            __syncthreads();  // this step's activations are in LDS; the other buffer is read
+            if (b + KB < b1) issue_a(b + KB, buf ^ 1);
+            load_d(b + KB, dnxt);
+#pragma unroll
+            for (int kb = 0; kb < KB; kb++) {
+                block(buf, kb);
+                load_b(b + KB, kb);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) dcur[nt] = dnxt[nt];
+        }
+    }
+
+    // epilogue: acc[mt][nt][i] is C[row][col] before the row's unscale (row 8 (i / 4) + 4 (l / 32) + i % 4 and
+    // column l % 32 of the tile)
+    const int N = W.rows;
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+        const int r0 = rowt + mt * 32 + 4 * (l >> 5);
+        float us[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) us[i] = unscale[r0 + 8 * (i >> 2) + (i & 3)];
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+            const int col = 16 * tilet + nt * 32 + (l & 31);
+            if (EPI == EPI_SWIGLU) {
+                // the gate/up matrix's rows 2j, 2j+1 are gate_j, up_j: columns 2j and 2j+1 of C lie in
+                // lanes c and c + 1 of a tile; the even lane writes h[row][j] = silu(gate) * up with
+                // the reference's SiLU of element row * F + j of the m x F array (silu_mul_kernel)
+                const int F = N >> 1;
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int row = r0 + 8 * (i >> 2) + (i & 3);
+                    const float y = acc[mt][nt][i] * us[i];
                     const float up = __shfl_xor(y, 1);
-                    if (!(c & 1) && col + 1 < N && row < m) {
+                    if (!(l & 1) && col + 1 < N && row < m) {
                         const int j = col >> 1;
                         C[(size_t)row * ldc + j] = silu_at(y, (size_t)row * F + j, (size_t)m * F) * up;
                     }
                 }
-        }
-        return;
-    }
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-        const int col = 16 * (tilet + wn * NT + nt) + c;
-        if (tilet + wn * NT + nt >= W.tiles || col >= N) continue;
-        const float bias = EPI == EPI_BIAS ? aux[col] : 0.0f;
-        float old[MT][4];
-        if (EPI == EPI_RESID) {
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int row = rowt + wm * 16 * MT + 16 * mt + 4 * G + i;
-                    old[mt][i] = row < m ? C[(size_t)row * ldc + col] : 0.0f;
-                }
-        }
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int row = rowt + wm * 16 * MT + 16 * mt + 4 * G + i;
-                if (row >= m) continue;
-                const float y = acc[mt][nt][i] * us[mt][i];
-                C[(size_t)row * ldc + col] = EPI == EPI_RESID ? old[mt][i] + y : y + bias;
+                continue;
             }
+            if (col >= N) continue;
+            const float bias = EPI == EPI_BIAS ? aux[col] : 0.0f;
+            float old[16];
+            if (EPI == EPI_RESID) {
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int row = r0 + 8 * (i >> 2) + (i & 3);
+                    old[i] = row < m ? C[(size_t)row * ldc + col] : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int row = r0 + 8 * (i >> 2) + (i & 3);
+                if (row >= m) continue;
+                const float y = acc[mt][nt][i] * us[i];
+                C[(size_t)row * ldc + col] = EPI == EPI_RESID ? old[i] + y : y + bias;
+            }
+        }
     }
 }
 
@@ -595,10 +528,9 @@ int mfma_rows_padded(int m) { return (m + GM_TILE - 1) / GM_TILE * GM_TILE; }
 
 // ---------------------------------------------------------------- split over K
 //
-// A grid of fewer workgroups than CUs (the small matrices of a short prompt) leaves most of
-// the chip idle and each wave walking a long chain of blocks alone.  Such a GEMM runs as Z
-// slices of K (gridDim.z), each writing its partial sums [z][m][N] (plain stores), then
-// gemm_ksum_kernel adds the partials in slice order and applies the epilogue: the same
+// A grid that leaves CUs idle or with one workgroup, walking a long chain of blocks alone,
+// runs as Z slices of K (gridDim.y), each writing its partial sums [z][m][N] (plain stores),
+// then gemm_ksum_kernel adds the partials in slice order and applies the epilogue: the same
 // result for every run, whatever order the slices finish in.
 
 static constexpr int KSPLIT_MAX = 8;         // slices
@@ -627,52 +559,45 @@ __global__ __launch_bounds__(256) void gemm_ksum_kernel(const float* __restrict_
         *c = y;
 }
 
-template <int MT, int NT, int S>
-static size_t g2_lds() {
-    return (size_t)S * sizeof(G2Stage<MT, NT>);
+template <int MT>
+static constexpr size_t gm_lds() {
+    return (size_t)2 * 2 * (2 * MT) * GM_KB * 1024;  // two steps of both parts
 }
 
-template <int MT, int NT, int S>
-static void gemm2_launch(const Q8MfmaDev& W, int m, const _Float16* hi, const _Float16* lo, const float* unscale,
-                         float* C, int ldc, const float* aux, Epi epi, hipStream_t st, int Z = 1) {
-    const dim3 grid((unsigned)(mfma_rows_padded(m) / (32 * MT)), (unsigned)((W.tiles + 2 * NT - 1) / (2 * NT)),
-                    (unsigned)Z);
+template <int MT, int NT>
+static void gemm_launch(const Q8MfmaDev& W, int m, const _Float16* hi, const _Float16* lo, const float* unscale,
+                        float* C, int ldc, const float* aux, Epi epi, hipStream_t st, int nbz) {
+    const int mtiles = (m + 32 * MT - 1) / (32 * MT), total = mtiles * ((W.tiles + 8 * NT - 1) / (8 * NT));
+    const dim3 grid((unsigned)total, (unsigned)((W.nb + nbz - 1) / nbz));
     const int K = W.nb * 32;
-    const size_t lds = g2_lds<MT, NT, S>();
+#define JY_GM(E)                                                                                                     \
+    hipLaunchKernelGGL((gemm_q8_mfma_kernel<E, MT, NT>), grid, dim3(256), gm_lds<MT>(), st, W, m, K, mtiles, total, \
+                       nbz, hi, lo, unscale, C, ldc, aux)
     switch (epi) {
-        case EPI_BIAS:
-            hipLaunchKernelGGL((gemm_q8_mfma2_kernel<EPI_BIAS, MT, NT, S>), grid, dim3(256), lds, st, W, m, K, hi, lo,
-                               unscale, C, ldc, aux);
-            break;
-        case EPI_RESID:
-            hipLaunchKernelGGL((gemm_q8_mfma2_kernel<EPI_RESID, MT, NT, S>), grid, dim3(256), lds, st, W, m, K, hi, lo,
-                               unscale, C, ldc, aux);
-            break;
-        case EPI_SWIGLU:
-            hipLaunchKernelGGL((gemm_q8_mfma2_kernel<EPI_SWIGLU, MT, NT, S>), grid, dim3(256), lds, st, W, m, K, hi, lo,
-                               unscale, C, ldc, aux);
-            break;
-        default:
-            hipLaunchKernelGGL((gemm_q8_mfma2_kernel<EPI_STORE, MT, NT, S>), grid, dim3(256), lds, st, W, m, K, hi, lo,
-                               unscale, C, ldc, aux);
-            break;
+        case EPI_BIAS: JY_GM(EPI_BIAS); break;
+        case EPI_RESID: JY_GM(EPI_RESID); break;
+        case EPI_SWIGLU: JY_GM(EPI_SWIGLU); break;
+        default: JY_GM(EPI_STORE); break;
     }
+#undef JY_GM
 }
 
-template <int MT, int NT, int S>
-static hipError_t gemm2_attr() {
+template <int MT, int NT>
+static hipError_t gemm_attr() {
     hipError_t e = hipSuccess;
-    for (const void* f : {reinterpret_cast<const void*>(&gemm_q8_mfma2_kernel<EPI_STORE, MT, NT, S>),
-                          reinterpret_cast<const void*>(&gemm_q8_mfma2_kernel<EPI_BIAS, MT, NT, S>),
-                          reinterpret_cast<const void*>(&gemm_q8_mfma2_kernel<EPI_RESID, MT, NT, S>),
-                          reinterpret_cast<const void*>(&gemm_q8_mfma2_kernel<EPI_SWIGLU, MT, NT, S>)})
-        if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)g2_lds<MT, NT, S>());
+    for (const void* f : {reinterpret_cast<const void*>(&gemm_q8_mfma_kernel<EPI_STORE, MT, NT>),
+                          reinterpret_cast<const void*>(&gemm_q8_mfma_kernel<EPI_BIAS, MT, NT>),
+                          reinterpret_cast<const void*>(&gemm_q8_mfma_kernel<EPI_RESID, MT, NT>),
+                          reinterpret_cast<const void*>(&gemm_q8_mfma_kernel<EPI_SWIGLU, MT, NT>)})
+        if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gm_lds<MT>());
     return e;
 }
 
 hipError_t gemm_mfma_init() {
-    hipError_t e = gemm2_attr<2, 8, 3>();
-    if (e == hipSuccess) e = gemm2_attr<2, 4, 3>();
+    hipError_t e = gemm_attr<1, 1>();
+    if (e == hipSuccess) e = gemm_attr<1, 2>();
+    if (e == hipSuccess) e = gemm_attr<2, 1>();
+    if (e == hipSuccess) e = gemm_attr<2, 2>();
     return e;
 }
 
@@ -690,48 +615,84 @@ static int gemm_cus() {
     return g_gemm_cus;
 }
 
-// workgroups of the wide tile's grid (128 columns per wave)
-static long wide_wgs(const Q8MfmaDev& W, int m) { return (long)(mfma_rows_padded(m) / 64) * ((W.tiles + 15) / 16); }
-
-// K slices for C = A W^T over m rows: 1 unless the narrow tile's grid has fewer workgroups
-// than CUs; then up to two workgroups per CU, at most KSPLIT_MAX slices of at least
-// KSPLIT_MIN_BLOCKS blocks, none of them empty.  (The SwiGLU epilogue pairs columns and is
-// not split.)
-int gemm_q8_mfma_ksplit(const Q8MfmaDev& W, int m, Epi epi) {
-    const int cus = gemm_cus();
-    const long wgs = (long)(mfma_rows_padded(m) / 64) * ((W.tiles + 7) / 8);
-    if (epi == EPI_SWIGLU || wide_wgs(W, m) >= 2L * cus || wgs >= cus) return 1;
-    const int z = (int)std::min<long>(std::min<long>(KSPLIT_MAX, 2L * cus / std::max(1L, wgs)),
-                                      W.nb / KSPLIT_MIN_BLOCKS);
-    if (z < 2) return 1;
-    const int nbz = (W.nb + z - 1) / z;
-    return (W.nb + nbz - 1) / nbz;
+// The K slices of C = A W^T over m rows.  For outputs of under 16 MiB as many as fill the chip
+// with two 64 x 128 tiles per CU, of at least KSPLIT_MIN_BLOCKS blocks, at most KSPLIT_MAX: the
+// more slices, the fewer additions in a row (4096 x 4096: error against 64 bits 2.1e-7 unsplit,
+// 1.3e-7 with 4), and the partial sums stay within 16 MiB, which callers with a small fixed
+// workspace need.  Larger ones have 1 to KSPLIT_MAX, by time (gemm_choice).  (The SwiGLU
+// epilogue pairs columns and is not split.)
+static int max_slices(const Q8MfmaDev& W, int m, Epi epi, bool& all) {
+    all = (size_t)m * W.rows * sizeof(float) < ((size_t)16 << 20);
+    if (epi == EPI_SWIGLU) return 1;
+    int z = std::min(KSPLIT_MAX, W.nb / KSPLIT_MIN_BLOCKS);
+    if (all) {
+        const int cus = gemm_cus(), tiles = (m + 127) / 128 * 2 * ((W.tiles + 7) / 8);
+        z = tiles >= cus ? 1 : std::min(z, 2 * cus / tiles);
+    }
+    return std::max(1, z);
 }
+
+// The tile (32 MT rows x 128 NT columns per workgroup) and the K slices of a launch: the least
+// of nbz blocks x max(lat, thr x the busiest CU's workgroups) ns, where lat is a lone
+// workgroup's time per block and thr the time per block and workgroup of a full CU, plus for
+// slices the partial sums' way through memory.  Measured at 28672 x 4096, 6144 x 4096, 4096 x
+// 4096, 4096 x 14336, 37888 x 3584, 9728 x 896, 1152 x 896 and 896 x 4864, 61 to 1024 rows.
+struct GmChoice {
+    int mt = 1, nt = 1, nbz = 0, z = 1;
+};
+static GmChoice gemm_choice(const Q8MfmaDev& W, int m, Epi epi, bool unsplit = false) {
+    struct Tile {
+        int mt, nt;
+        float lat, thr;
+    };
+    static constexpr Tile tiles[] = {{2, 2, 640.0f, 550.0f}, {1, 2, 400.0f, 305.0f}, {2, 1, 400.0f, 305.0f}, {1, 1, 275.0f, 170.0f}};
+    const int cus = gemm_cus();
+    bool all = false;
+    const int zmax = unsplit ? 1 : max_slices(W, m, epi, all);
+    GmChoice best;
+    float cost = 0.0f;
+    for (const Tile& t : tiles)
+        for (int zi = all ? zmax : 1; zi <= zmax; zi++) {
+            const int nbz = ((W.nb + zi - 1) / zi + GM_KB - 1) / GM_KB * GM_KB, z = (W.nb + nbz - 1) / nbz;
+            const long wgs = (long)((m + 32 * t.mt - 1) / (32 * t.mt)) * ((W.tiles + 8 * t.nt - 1) / (8 * t.nt)) * z;
+            float c = (float)nbz * std::max(t.lat, t.thr * (float)((wgs + cus - 1) / cus));
+            if (z > 1) c += 1500.0f + (float)z * (float)m * (float)W.rows * (8.0f / 4000.0f);
+            if (!best.nbz || c < cost) {
+                cost = c;
+                best.mt = t.mt, best.nt = t.nt, best.nbz = nbz, best.z = z;
+            }
+        }
+    return best;
+}
+
+int gemm_q8_mfma_ksplit(const Q8MfmaDev& W, int m, Epi epi) { return gemm_choice(W, m, epi).z; }
 
 size_t gemm_q8_mfma_kpart_floats(const Q8MfmaDev& W, int m, Epi epi) {
     const int z = gemm_q8_mfma_ksplit(W, m, epi);
     return z > 1 ? (size_t)z * m * W.rows : 0;
 }
 
-// the wide tile (128 columns per wave) when its grid gives every CU at least two
-// workgroups, else the narrow one (64 columns per wave, twice the workgroups), split over K
-// when even that grid leaves CUs idle and `kpart` holds the partials.  Measured at the
-// Llama-3-8B shapes and 1024 tokens (the activation split included): gate/up (28672 x
-// 4096) 576 us wide, 686 narrow; QKV 164, O 118, down 422 us narrow.
 int launch_gemm_q8_mfma(const Q8MfmaDev& W, int m, const _Float16* hi, const _Float16* lo, const float* unscale,
                         float* C, int ldc, const float* aux, Epi epi, hipStream_t st, float* kpart, size_t kpart_n,
                         bool defer) {
-    const int cus = gemm_cus();
-    if (wide_wgs(W, m) >= 2L * cus) {
-        gemm2_launch<2, 8, 3>(W, m, hi, lo, unscale, C, ldc, aux, epi, st);
+    GmChoice g = gemm_choice(W, m, epi);
+    if (g.z > 1 && (!kpart || (size_t)g.z * m * W.rows > kpart_n)) g = gemm_choice(W, m, epi, true);
+    const int Z = g.z;
+    auto run = [&](float* out, int ld, const float* ax, Epi e) {
+        if (g.mt == 2 && g.nt == 2)
+            gemm_launch<2, 2>(W, m, hi, lo, unscale, out, ld, ax, e, st, g.nbz);
+        else if (g.mt == 2)
+            gemm_launch<2, 1>(W, m, hi, lo, unscale, out, ld, ax, e, st, g.nbz);
+        else if (g.nt == 2)
+            gemm_launch<1, 2>(W, m, hi, lo, unscale, out, ld, ax, e, st, g.nbz);
+        else
+            gemm_launch<1, 1>(W, m, hi, lo, unscale, out, ld, ax, e, st, g.nbz);
+    };
+    if (Z < 2) {
+        run(C, ldc, aux, epi);
         return 0;
     }
-    const int Z = gemm_q8_mfma_ksplit(W, m, epi);
-    if (Z < 2 || !kpart || (size_t)Z * m * W.rows > kpart_n) {
-        gemm2_launch<2, 4, 3>(W, m, hi, lo, unscale, C, ldc, aux, epi, st);
-        return 0;
-    }
-    gemm2_launch<2, 4, 3>(W, m, hi, lo, unscale, kpart, W.rows, nullptr, EPI_STORE, st, Z);
+    run(kpart, W.rows, nullptr, EPI_STORE);
     if (defer) return Z;
     const size_t n = (size_t)m * W.rows;
     const dim3 grid((unsigned)((n + 255) / 256));

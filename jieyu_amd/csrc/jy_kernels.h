@@ -26,9 +26,10 @@ struct Q8Dev {
 
 // A Q8_0 matrix as the matrix-core prompt GEMM reads it (jy_gemm_mfma.hip): per tile of
 // 16 rows and block of 32 weights, 512 bytes in MFMA B-operand lane order (q), and the
-// block scales as fp32, four blocks of a row together (d).  Rows past `rows` are zero.
+// block scales as fp32, four blocks of a row together, zero past the last block (d).  Rows
+// past `rows` are zero.
 struct Q8MfmaDev {
-    int8_t* q = nullptr;  // [tiles][nb][64 lanes][8]
+    int8_t* q = nullptr;  // [tiles][nb][2 k halves][16 rows][16]
     float* d = nullptr;   // [tiles][nb4][16 rows][4]
     int rows = 0, cols = 0, nb = 0, nb4 = 0, tiles = 0;
 };

@@ -9,6 +9,7 @@ namespace jy {
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
+typedef float f16_t __attribute__((ext_vector_type(16)));
 typedef int i4_t __attribute__((ext_vector_type(4)));
 typedef int i2_t __attribute__((ext_vector_type(2)));
 
@@ -24,6 +25,16 @@ __device__ __forceinline__ h8_t q8_to_h8(uint32_t w0, uint32_t w1) {
     const h2_t r0 = __builtin_bit_cast(h2_t, p0) - off, r1 = __builtin_bit_cast(h2_t, p1) - off;
     const h2_t r2 = __builtin_bit_cast(h2_t, p2) - off, r3 = __builtin_bit_cast(h2_t, p3) - off;
     return h8_t{r0.x, r0.y, r1.x, r1.y, r2.x, r2.y, r3.x, r3.y};
+}
+
+// element e of v, e a constant after unrolling
+__device__ __forceinline__ float f4_get(const float4& v, int e) { return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w; }
+
+// blocks in launch order go round the 8 XCDs: give each XCD a contiguous run of tiles, so
+// that the row groups of one column tile share its L2
+__device__ __forceinline__ int xcd_tile(int id, int total) {
+    const int x = id & 7, q = total >> 3, r = total & 7;
+    return x * q + min(x, r) + (id >> 3);
 }
 
 }  // namespace jy

@@ -152,6 +152,31 @@ def test_mfma_gemm_within_tolerance(jy, oracle_lib, m, rows, cols):
         assert np.array_equal(tiles.view(np.uint32), ref.view(np.uint32))
 
 
+# the GEMM's tiles (32 or 64 rows x 128 or 256 columns, by rows and columns), block counts that
+# leave 1, 2 or 3 blocks of a step of four, one block alone, columns that end inside a 16-, 32-
+# and 128-column tile, slices of K with outputs under and over 16 MiB, and the activation split
+# of rows wider than 16384 values
+@pytest.mark.parametrize("m,rows,cols", [
+    (33, 130, 32), (31, 28679, 96), (61, 28672, 160), (100, 20011, 64), (300, 20000, 224), (1000, 12007, 96),
+    (1024, 4112, 1056), (1030, 4112, 4128), (40, 1000, 17024), (5, 77, 32768)])
+def test_mfma_gemm_tiles(jy, oracle_lib, m, rows, cols):
+    """as above: within 1e-5 of sum |a| |w| (22 significant bits of each activation, 2.4e-7, and
+    fp32 sums of at most cols / 32 + 64 terms in random order: a few 1e-6 of it)"""
+    from conftest import q8_random_uniform
+    say(f"mfma gemm tiles m={m} {rows}x{cols}")
+    w = q8_random_uniform(oracle_lib, rows, cols, seed=5)
+    A = np.zeros((m, cols), np.float32)
+    oracle_lib.jysyn_normal_fill(5, 19, 1.0, ptr(A), A.size)
+    M = jy.Q8Matrix(w, rows, cols)
+    M.set_mode(jy.MODE_MFMA_PREFILL)
+    got = M.gemm(A)
+    M.close()
+    wf = dequant(w, rows, cols)
+    A64 = A.astype(np.float64)
+    bound = 1e-5 * (np.abs(A64) @ np.abs(wf).T)
+    assert np.all(np.abs(got - A64 @ wf.T) <= bound)
+
+
 MODES = {"SPLIT_ATTN": 1, "SPLIT_MV": 2, "MFMA_PREFILL": 4, "FAST": 7, "PERSIST": 7 | 8}
 
 
