@@ -60,10 +60,10 @@ __global__ __launch_bounds__(64 * WW) __attribute__((amdgpu_waves_per_eu(4, 4)))
 // range as one slice, the other rows' later keys masked per query column; the normalised
 // output straight to a.out; row groups in descending order (the longest first).  R rows
 // fill the 8 query columns of the slice's matrix operations (R x the group's heads).
-template <int P, int R>
-__global__ __launch_bounds__(SPL_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void attn_prefill_kernel(AttnArgs a) {
-    __shared__ MslLds<P * 16, 4> lds;
-    attn_slice_mfma<P, SPL_GMAX, 4, false, 1, 1, R>(a, 1, nullptr, blockIdx.x, 0, lds,
+template <int P, int R, int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, 4))) void attn_prefill_kernel(AttnArgs a) {
+    __shared__ MslLds<P * 16, NW> lds;
+    attn_slice_mfma<P, SPL_GMAX, NW, false, 1, 1, R>(a, 1, nullptr, blockIdx.x, 0, lds,
                                                     a.nrows - 1 - R * (int)blockIdx.y);
 }
 
@@ -202,22 +202,41 @@ void launch_attention_whole(const AttnArgs& a, hipStream_t st) {
 
 // Rows per workgroup: as many as the 8 query columns hold (R = 8 / split_heads(G)).
 // Llama-3-8B shape (4 query heads per kv head), 1024 prompt rows: one row per workgroup
-// 108 us per layer, two rows [measured below].
-void launch_attention_prefill_split(const AttnArgs& a, hipStream_t st) {
-    const int R = SPL_GMAX / split_heads(a.nh / a.nkv);
-    const dim3 grid(a.nkv, (a.nrows + R - 1) / R), block(SPL_THREADS);
-    auto k = attn_prefill_kernel<8, 1>;
+// 104 us per layer, two rows 64.
+//
+// Waves per workgroup: a short chunk over a long cache has one workgroup per CU or fewer, and
+// with 4 waves each a CU waits on the loads of 4.  Grids of up to two workgroups per CU take 8
+// waves from 512 keys, of up to one 16 waves from 2048 (below, the merge of more waves costs
+// what their loads gain).  Per layer, 4 waves -> now: 61 rows x 5000 keys, Qwen2.5-7B heads
+// 50.2 -> 36.8 us (the keys and values through L2 at 9 TB/s), Llama-3-8B heads 54.6 -> 45.3; 61 x
+// 700 13.5 -> 11.2; 100 x 3000, Qwen2.5-0.5B heads 25.0 -> 18.0; 30 x 1000 11.8 -> 9.2.
+template <int NW>
+static void prefill_launch(const AttnArgs& a, int R, hipStream_t st) {
+    const dim3 grid(a.nkv, (a.nrows + R - 1) / R), block(64 * NW);
+    auto k = attn_prefill_kernel<8, 1, NW>;
     switch (R * (a.hd == 64 ? -1 : 1)) {
-        case -1: k = attn_prefill_kernel<4, 1>; break;
-        case -2: k = attn_prefill_kernel<4, 2>; break;
-        case -4: k = attn_prefill_kernel<4, 4>; break;
-        case -8: k = attn_prefill_kernel<4, 8>; break;
-        case 2: k = attn_prefill_kernel<8, 2>; break;
-        case 4: k = attn_prefill_kernel<8, 4>; break;
-        case 8: k = attn_prefill_kernel<8, 8>; break;
+        case -1: k = attn_prefill_kernel<4, 1, NW>; break;
+        case -2: k = attn_prefill_kernel<4, 2, NW>; break;
+        case -4: k = attn_prefill_kernel<4, 4, NW>; break;
+        case -8: k = attn_prefill_kernel<4, 8, NW>; break;
+        case 2: k = attn_prefill_kernel<8, 2, NW>; break;
+        case 4: k = attn_prefill_kernel<8, 4, NW>; break;
+        case 8: k = attn_prefill_kernel<8, 8, NW>; break;
         default: break;
     }
     hipLaunchKernelGGL(k, grid, block, 0, st, a);
+}
+
+void launch_attention_prefill_split(const AttnArgs& a, hipStream_t st) {
+    const int R = SPL_GMAX / split_heads(a.nh / a.nkv);
+    const long wgs = (long)a.nkv * ((a.nrows + R - 1) / R);
+    const int keys = a.start_pos + a.row0 + a.nrows;
+    if (wgs <= 256 && keys >= 2048)
+        prefill_launch<16>(a, R, st);
+    else if (wgs <= 512 && keys >= 512)
+        prefill_launch<8>(a, R, st);
+    else
+        prefill_launch<4>(a, R, st);
 }
 
 }  // namespace jy

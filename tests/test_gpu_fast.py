@@ -177,6 +177,36 @@ def test_mfma_gemm_tiles(jy, oracle_lib, m, rows, cols):
     assert np.all(np.abs(got - A64 @ wf.T) <= bound)
 
 
+# a chunk of prompt rows over a cached range: 4, 8 or 16 waves per workgroup by rows and keys
+# (their limits 512 and 2048 keys, 256 and 512 workgroups), key counts that leave waves without
+# a step, both head sizes, one and several rows per workgroup
+@pytest.mark.parametrize("heads,kv,hd", [(4, 2, 64), (14, 2, 128), (8, 2, 128)])
+@pytest.mark.parametrize("rows,past", [(5, 506), (5, 507), (3, 2044), (3, 2045), (130, 2100), (270, 600), (2, 3000)])
+def test_prompt_attention_waves(jy, oracle_lib, heads, kv, hd, rows, past):
+    """the split attention against the exact mode (itself bit-equal to the oracle's) on the same
+    cache and rows, within the tolerance mode's 1e-3 of the outputs' largest value"""
+    say(f"prompt attention {heads}/{kv}x{hd} rows {rows} past {past}")
+    cfg = dict(name="llama3-8b", num_layers=1, hidden=256, num_heads=heads, num_kv_heads=kv, head_dim=hd,
+               intermediate=256, vocab_size=64)
+    from jieyu_amd.model import Synth, synth_config
+    s = Synth(oracle_lib, synth_config(cfg.pop("name"), **cfg))
+    rng = np.random.default_rng(rows + past)
+    X = rng.standard_normal((rows, 256)).astype(np.float32)
+    k, v = [rng.integers(-127, 128, (past, kv, hd)).astype(np.int8) for _ in range(2)]
+    ks, vs = [rng.uniform(0.005, 0.03, (past, kv)).astype(np.float32) for _ in range(2)]
+    out = []
+    for mode in (jy.MODE_EXACT, 1):  # (1: the split attention alone)
+        g = jy.GpuModel(s.desc, past + rows)
+        g.mode = mode
+        c = g.kv()
+        c.write(0, 0, k, ks, v, vs)
+        out.append(g.forward_cached(c, X, past))
+        c.close()
+        g.close()
+    s.close()
+    assert np.max(np.abs(out[1] - out[0])) <= 1e-3 * np.max(np.abs(out[0]))
+
+
 MODES = {"SPLIT_ATTN": 1, "SPLIT_MV": 2, "MFMA_PREFILL": 4, "FAST": 7, "PERSIST": 7 | 8}
 
 
