@@ -118,6 +118,11 @@ JYHIP_API int jyhip_kv_read(const jyhip_kv* kv, int layer, int pos0, int npos, i
 JYHIP_API int jyhip_forward_cached(jyhip_model* model, jyhip_kv* kv, float* X, int seq, int start_pos,
                                    float* layer_out);
 
+/* The same with the hidden states to `out` (host [seq][hidden], X itself or apart from it),
+ * for a caller that keeps X or would copy it only to have it overwritten. */
+JYHIP_API int jyhip_forward_cached_to(jyhip_model* model, jyhip_kv* kv, const float* X, float* out, int seq,
+                                      int start_pos, float* layer_out);
+
 /* Bytes of the static per-GPU workspace of jyhip_forward_cached_noalloc. */
 #define JYHIP_NOALLOC_SCRATCH_BYTES (16u << 20)
 

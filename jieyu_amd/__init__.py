@@ -76,6 +76,7 @@ def lib():
     _proto(L, "jyhip_kv_write", I, P, I, I, I, P, P, P, P)
     _proto(L, "jyhip_kv_read", I, P, I, I, I, P, P, P, P)
     _proto(L, "jyhip_forward_cached", I, P, P, P, I, I, P)
+    _proto(L, "jyhip_forward_cached_to", I, P, P, P, P, I, I, P)
     _proto(L, "jyhip_forward_cached_noalloc", I, P, P, P, I, I)
     _proto(L, "jyhip_generate", I, P, P, P, I, P, I, I, I, F, F, P, TOKEN_CB, P, P, C.POINTER(Stats))
     _proto(L, "jyhip_session_begin", P, P, P, P, I, P, I, I, I, F, F)
@@ -204,11 +205,12 @@ class GpuModel:
 
     def forward_cached(self, kv, X, start_pos, layer_out=False):
         """forward_cached: X [seq][hidden] float32 -> final-normed states (new array)."""
-        X = np.array(X, np.float32, copy=True, order="C")
+        X = np.asarray(X, np.float32, order="C")
+        out = np.empty(X.shape, np.float32)
         seq = X.shape[0]
         lo = np.zeros((self.num_layers, seq, self.hidden), np.float32) if layer_out else None
-        _check(self._lib.jyhip_forward_cached(self.h, kv.h, _ptr(X), seq, start_pos, _ptr(lo)))
-        return (X, lo) if layer_out else X
+        _check(self._lib.jyhip_forward_cached_to(self.h, kv.h, _ptr(X), _ptr(out), seq, start_pos, _ptr(lo)))
+        return (out, lo) if layer_out else out
 
     def forward_cached_noalloc(self, kv, X, start_pos):
         """forward_cached over the GPU's static workspace (jyhip_forward_cached_noalloc)."""

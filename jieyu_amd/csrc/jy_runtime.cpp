@@ -16,6 +16,7 @@
 
 #include "jieyu_amd.h"
 #include "jy_kernels.h"
+#include "jy_stage.h"
 
 using namespace jy;
 
@@ -162,6 +163,7 @@ struct jyhip_model {
     size_t pk_flag_bytes = 0;
     int* pk_err = nullptr;         // set by the kernel when a barrier wait gave up
     size_t pk_lds = 0;
+    HostStage stage;  // forward calls' rows in and out (where it has no ring: plain copies)
     std::vector<void*> owned;
 };
 
@@ -675,6 +677,7 @@ void upload(jyhip_model* m, const jy_model_desc* d, int max_seq, int wtype) {
     m->max_seq = max_seq;
     m->theta = d->rope_theta;
     CK(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
+    (void)m->stage.init();
 
     std::vector<float> c, s;
     rope_table(max_seq, m->hd, m->theta, c, s);
@@ -788,6 +791,7 @@ void release(jyhip_model* m) {
                     (void*)w.q8, (void*)w.qsc, (void*)w.scores, (void*)w.part, (void*)w.ah, (void*)w.al,
                     (void*)w.aus, (void*)w.kp})
         dfree(p);
+    m->stage.release();
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
 }
@@ -1548,8 +1552,33 @@ int generate_impl(jyhip_model* m, jyhip_kv* kv_in, const int* prompt, int plen, 
 }
 
 
-int forward_impl(jyhip_model* m, jyhip_kv* kv, float* X, int seq, int start_pos, float* layer_out) {
-    if (!kv || !X) fail("forward: NULL kv or X");
+// a forward call's rows into w.X, and the final RMSNorm (forward.h:86-94) of w.X's rows to the
+// caller, the stream waited for
+void rows_in(jyhip_model* m, Workspace& w, const float* X, int seq) {
+    const size_t n = sizeof(float) * seq * m->H;
+    if (m->stage.ready())
+        CK(m->stage.to_device(w.X, X, n, m->stream));
+    else
+        CK(hipMemcpyAsync(w.X, X, n, hipMemcpyHostToDevice, m->stream));
+}
+
+void rows_out(jyhip_model* m, Workspace& w, float* out, int seq) {
+    hipStream_t st = m->stream;
+    const size_t row = sizeof(float) * m->H;
+    if (m->stage.ready() && row <= HostStage::SLOT) {  // the norm writes the pinned ring itself
+        CK(m->stage.to_host(out, seq, row, st, [&](size_t r0, size_t n, void* p) {
+            launch_rmsnorm(w.X + r0 * m->H, static_cast<float*>(p), m->final_rms, m->H, (int)n, st);
+        }));
+        return;
+    }
+    launch_rmsnorm(w.X, w.xn, m->final_rms, m->H, seq, st);
+    CK(hipGetLastError());
+    CK(hipMemcpyAsync(out, w.xn, row * seq, hipMemcpyDeviceToHost, st));
+    CK(hipStreamSynchronize(st));
+}
+
+int forward_impl(jyhip_model* m, jyhip_kv* kv, const float* X, float* out, int seq, int start_pos, float* layer_out) {
+    if (!kv || !X || !out) fail("forward: NULL kv or X");
     if (kv->dev.num_layers < m->L || kv->dev.nkv != m->nkv || kv->dev.hd != m->hd)
         fail("forward: KV cache shape does not match the model");  // forward.h:60-61
     if (kv->device != m->device) fail("forward: the KV cache is on another device than the model");
@@ -1557,18 +1586,14 @@ int forward_impl(jyhip_model* m, jyhip_kv* kv, float* X, int seq, int start_pos,
     if (seq <= 0) fail("forward: seq must be positive");
     if ((size_t)start_pos + seq > (size_t)kv->dev.max_seq) fail("forward: KV cache capacity exceeded");
     if (start_pos + seq > m->max_seq) fail("forward: position beyond the RoPE table");
-    hipStream_t st = m->stream;
     const int max_keys = (start_pos + seq + 3) / 4 * 4;
     ensure_ws(m, seq);
     ensure_scores(m, scores_need(m, seq, max_keys));
     ensure_part(m, part_need(m, max_keys));
     Workspace& w = m->ws;
-    CK(hipMemcpyAsync(w.X, X, sizeof(float) * seq * m->H, hipMemcpyHostToDevice, st));
+    rows_in(m, w, X, seq);
     run_layers(m, w, kv->dev, seq, start_pos, nullptr, layer_out, max_keys);
-    launch_rmsnorm(w.X, w.xn, m->final_rms, m->H, seq, st);  // forward.h:86-94
-    CK(hipGetLastError());
-    CK(hipMemcpyAsync(X, w.xn, sizeof(float) * seq * m->H, hipMemcpyDeviceToHost, st));
-    CK(hipStreamSynchronize(st));
+    rows_out(m, w, out, seq);
     check_persist(m);
     kv->current_len = start_pos + seq;
     return 0;
@@ -1634,16 +1659,12 @@ int forward_noalloc(jyhip_model* m, jyhip_kv* kv, float* X, int seq, int start_p
         fail("forward_cached_noalloc: " + std::to_string(seq) + " rows attending " + std::to_string(start_pos + seq) +
              " keys need " + std::to_string(need) + " bytes of workspace, more than the " +
              std::to_string((size_t)JYHIP_NOALLOC_SCRATCH_BYTES) + "-byte static scratch");
-    hipStream_t st = m->stream;
     // the allocating path starts from zeroed buffers; so does this one, whatever an
     // earlier call left in the shared array
-    launch_zero_fill(base, need, st);
-    CK(hipMemcpyAsync(w.X, X, sizeof(float) * seq * m->H, hipMemcpyHostToDevice, st));
+    launch_zero_fill(base, need, m->stream);
+    rows_in(m, w, X, seq);
     run_layers(m, w, kv->dev, seq, start_pos, nullptr, nullptr, max_keys);
-    launch_rmsnorm(w.X, w.xn, m->final_rms, m->H, seq, st);  // forward.h:86-94
-    CK(hipGetLastError());
-    CK(hipMemcpyAsync(X, w.xn, sizeof(float) * seq * m->H, hipMemcpyDeviceToHost, st));
-    CK(hipStreamSynchronize(st));
+    rows_out(m, w, X, seq);
     check_persist(m);
     kv->current_len = start_pos + seq;
     return 0;
@@ -1835,7 +1856,15 @@ JYHIP_API int jyhip_kv_read(const jyhip_kv* kv, int layer, int pos0, int npos, i
 JYHIP_API int jyhip_forward_cached(jyhip_model* m, jyhip_kv* kv, float* X, int seq, int start_pos, float* layer_out) {
     return guarded([&]() {
         if (!m) fail("model is NULL");
-        return forward_impl(m, kv, X, seq, start_pos, layer_out);
+        return forward_impl(m, kv, X, X, seq, start_pos, layer_out);
+    }, -1);
+}
+
+JYHIP_API int jyhip_forward_cached_to(jyhip_model* m, jyhip_kv* kv, const float* X, float* out, int seq, int start_pos,
+                                      float* layer_out) {
+    return guarded([&]() {
+        if (!m) fail("model is NULL");
+        return forward_impl(m, kv, X, out, seq, start_pos, layer_out);
     }, -1);
 }
 
