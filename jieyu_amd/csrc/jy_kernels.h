@@ -139,6 +139,14 @@ void launch_matvec_f32(const float* B, int K, int N, const float* x, float* out,
                        hipStream_t st);
 void launch_matvec_f16(const uint16_t* B, int K, int N, const float* x, float* out, const float* aux, Epi epi,
                        hipStream_t st);
+// decode of dense models with fewer launches: n <= 3 f32 or f16 matrices (panels, `type`) of one
+// RMS-normalised row (weights nw; only where dense_norm_fits(K)), out[i] = B[i] norm(x) (+ aux[i]);
+// and the down projection with SiLU, X += B (silu(gate) * up)
+bool dense_norm_fits(int K);
+void launch_dense_norm(int type, const void* const* B, const int* N, float* const* out, const float* const* aux, int n,
+                       int K, const float* x, const float* nw, hipStream_t st);
+void launch_dense_down(int type, const void* B, int K, int N, const float* gate, const float* up, float* X,
+                       hipStream_t st);
 // prefill GEMMs, C[m][N] (+ epilogue: EPI_STORE / EPI_BIAS / EPI_RESID)
 void launch_gemm_q8(const Q8Dev& W, int m, const float* A, float* C, const float* aux, Epi epi, hipStream_t st);
 // the matrix-core form (jy_gemm_mfma.hip): the copy of W it reads (built once), the split

@@ -881,15 +881,27 @@ void run_decode_layers(jyhip_model* m, Workspace& w, const KVDev& kv, const int*
             qa.nh = m->nh;
             qa.nkv = m->nkv;
             qa.hd = m->hd;
+            // (n matrices of one dense type, D.w's index i[])
+            auto dense = [&](std::initializer_list<int> i) {
+                for (int k : i)
+                    if (!D.w[k].dense || D.w[k].type != D.w[*i.begin()].type) return false;
+                return true;
+            };
             if (launch_mv_qkv(D.w, w.X, D.rms1, w.qkv, qa, st)) {
                 at.fused = true;
                 at.qkv = w.qkv;
             } else {
-                const Epi qe = D.bqkv ? EPI_BIAS : EPI_STORE;
-                launch_rmsnorm(w.X, w.xn, D.rms1, H, 1, st);
-                launch_mv(D.w[0], w.xn, w.qkv, qe, D.bqkv, st);
-                launch_mv(D.w[1], w.xn, w.qkv + qd, qe, D.bqkv ? D.bqkv + qd : nullptr, st);
-                launch_mv(D.w[2], w.xn, w.qkv + qd + kvd, qe, D.bqkv ? D.bqkv + qd + kvd : nullptr, st);
+                const float* aux[3] = {D.bqkv, D.bqkv ? D.bqkv + qd : nullptr, D.bqkv ? D.bqkv + qd + kvd : nullptr};
+                float* out[3] = {w.qkv, w.qkv + qd, w.qkv + qd + kvd};
+                if (dense({0, 1, 2}) && dense_norm_fits(H)) {
+                    const void* B[3] = {D.w[0].dense, D.w[1].dense, D.w[2].dense};
+                    const int N[3] = {qd, kvd, kvd};
+                    launch_dense_norm(D.w[0].type, B, N, out, aux, 3, H, w.X, D.rms1, st);
+                } else {
+                    launch_rmsnorm(w.X, w.xn, D.rms1, H, 1, st);
+                    for (int i = 0; i < 3; i++)
+                        launch_mv(D.w[i], w.xn, out[i], aux[i] ? EPI_BIAS : EPI_STORE, aux[i], st);
+                }
                 launch_rope_pack(w.qkv, 1, pos0, state, m->nh, m->nkv, m->hd, m->cos_t, m->sin_t, kv, l, w.q8, w.qsc,
                                  st);
                 at.fused = false;
@@ -899,16 +911,32 @@ void run_decode_layers(jyhip_model* m, Workspace& w, const KVDev& kv, const int*
             }
             launch_attention(at, st);
             launch_mv(D.w[3], w.att, w.X, EPI_RESID, nullptr, st);
-            if (!launch_mv_gate_up(D.w[4], D.w[6], w.X, D.rms2, w.h, st)) {
+            const bool fused_h = launch_mv_gate_up(D.w[4], D.w[6], w.X, D.rms2, w.h, st);
+            if (!fused_h && dense({4, 6}) && dense_norm_fits(H)) {
+                const void* B[2] = {D.w[4].dense, D.w[6].dense};
+                const int N[2] = {F, F};
+                float* out[2] = {w.g, w.u};
+                launch_dense_norm(D.w[4].type, B, N, out, nullptr, 2, H, w.X, D.rms2, st);
+            } else if (!fused_h) {
                 launch_rmsnorm(w.X, w.xn, D.rms2, H, 1, st);
                 launch_mv(D.w[4], w.xn, w.g, EPI_STORE, nullptr, st);
                 launch_mv(D.w[6], w.xn, w.u, EPI_STORE, nullptr, st);
-                launch_silu_mul(w.g, w.u, 0, 1, F, w.h, st);
             }
-            launch_mv(D.w[5], w.h, w.X, EPI_RESID, nullptr, st);
+            if (!fused_h && dense({5})) {
+                launch_dense_down(D.w[5].type, D.w[5].dense, F, H, w.g, w.u, w.X, st);
+            } else {
+                if (!fused_h) launch_silu_mul(w.g, w.u, 0, 1, F, w.h, st);
+                launch_mv(D.w[5], w.h, w.X, EPI_RESID, nullptr, st);
+            }
         } else {
-            launch_rmsnorm(w.X, w.xn, D.rms1, H, 1, st);
-            launch_matvec_f32(D.f_qkv, H, NQ, w.xn, w.qkv, D.bqkv, D.bqkv ? EPI_BIAS : EPI_STORE, st);
+            const bool fits = dense_norm_fits(H);
+            if (fits) {
+                const void* B = D.f_qkv;
+                launch_dense_norm(JY_F32, &B, &NQ, &w.qkv, &D.bqkv, 1, H, w.X, D.rms1, st);
+            } else {
+                launch_rmsnorm(w.X, w.xn, D.rms1, H, 1, st);
+                launch_matvec_f32(D.f_qkv, H, NQ, w.xn, w.qkv, D.bqkv, D.bqkv ? EPI_BIAS : EPI_STORE, st);
+            }
             launch_rope_pack(w.qkv, 1, pos0, state, m->nh, m->nkv, m->hd, m->cos_t, m->sin_t, kv, l, w.q8, w.qsc, st);
             at.fused = false;
             at.q8 = w.q8;
@@ -916,10 +944,17 @@ void run_decode_layers(jyhip_model* m, Workspace& w, const KVDev& kv, const int*
             at.row0 = 0;
             launch_attention(at, st);
             launch_matvec_f32(D.f_o, m->qd, H, w.att, w.X, nullptr, EPI_RESID, st);
-            launch_rmsnorm(w.X, w.xn, D.rms2, H, 1, st);
-            launch_matvec_f32(D.f_w1, H, F, w.xn, w.g, nullptr, EPI_STORE, st);
-            launch_matvec_f32(D.f_w3, H, F, w.xn, w.h, w.g, EPI_SWIGLU, st);  // h = silu(gate) * up
-            launch_matvec_f32(D.f_w2, F, H, w.h, w.X, nullptr, EPI_RESID, st);
+            if (fits) {
+                const void* B[2] = {D.f_w1, D.f_w3};
+                const int N[2] = {F, F};
+                float* out[2] = {w.g, w.u};
+                launch_dense_norm(JY_F32, B, N, out, nullptr, 2, H, w.X, D.rms2, st);
+            } else {
+                launch_rmsnorm(w.X, w.xn, D.rms2, H, 1, st);
+                launch_matvec_f32(D.f_w1, H, F, w.xn, w.g, nullptr, EPI_STORE, st);
+                launch_matvec_f32(D.f_w3, H, F, w.xn, w.u, nullptr, EPI_STORE, st);
+            }
+            launch_dense_down(JY_F32, D.f_w2, F, H, w.g, w.u, w.X, st);  // (silu(gate) * up in the load)
         }
         if (layer_out_host) {
             CK(hipMemcpyAsync(layer_out_host + (size_t)l * H, w.X, sizeof(float) * H, hipMemcpyDeviceToHost, st));
@@ -1092,8 +1127,16 @@ void final_and_head(jyhip_model* m, Workspace& w, const float* xlast, bool argma
         q8_matvec(m, m->lm_q8, xlast, m->final_rms, m->logits, argmax ? EPI_ARGMAX : EPI_STORE, a, m->stream);
     } else if (m->wtype == WT_MIXED) {
         if (launch_mv_norm(m->lm_w, xlast, m->final_rms, m->logits, m->stream)) return;
+        if (m->lm_w.dense && dense_norm_fits(m->H)) {
+            launch_dense_norm(m->lm_w.type, &m->lm_w.dense, &m->V, &m->logits, nullptr, 1, m->H, xlast, m->final_rms,
+                              m->stream);
+            return;
+        }
         launch_rmsnorm(xlast, w.xn, m->final_rms, m->H, 1, m->stream);
         launch_mv(m->lm_w, w.xn, m->logits, EPI_STORE, nullptr, m->stream);
+    } else if (dense_norm_fits(m->H)) {
+        const void* B = m->lm_f32;
+        launch_dense_norm(JY_F32, &B, &m->V, &m->logits, nullptr, 1, m->H, xlast, m->final_rms, m->stream);
     } else {
         launch_rmsnorm(xlast, w.xn, m->final_rms, m->H, 1, m->stream);
         launch_matvec_f32(m->lm_f32, m->H, m->V, w.xn, m->logits, nullptr, EPI_STORE, m->stream);

@@ -116,6 +116,42 @@ def test_kquant_groups_that_do_not_fuse(jy, oracle_lib, wv, w3):
                 embed=QM.JY_Q6_K, lm=QM.JY_Q4_K, tied=False)
     check_forward(jy, oracle_lib, spec, (1, 1, 2, 1))
 
+def check_generate(jy, oracle_lib, spec):
+    """greedy picks and the last logits against the oracle's"""
+    QM.SPECS["edge"] = spec
+    try:
+        m = QM.build_model("edge", 3)
+    finally:
+        del QM.SPECS["edge"]
+    d, keep = QM.desc_of(m)
+    cos, sin = rope_tables(oracle_lib, 16, spec["hd"], d.rope_theta)
+    prompt = QM.prompt_of(m, 3)
+    want, wl = np.zeros(17, np.int32), np.zeros(spec["vocab"], np.float32)
+    n = oracle_lib.jyo_generate(C.byref(d), ptr(prompt), 3, None, 0, ptr(cos), ptr(sin), 16, 4, 0.0, 1.0, ptr(want),
+                                None, ptr(wl))
+    g = jy.GpuModel(d, 16)
+    ids, _, logits = g.generate(prompt, 4, want_logits=True)
+    g.close()
+    assert ids.tolist() == want[:n].tolist()
+    assert bits_equal(logits, wl)
+
+
+# dense decode: the launches with RMSNorm (q/k/v, gate/up, the head) and with SiLU (down) at input
+# widths under, at and over one block of the panel (256 f32, 512 f16 rows), not a multiple of a
+# 16-byte piece, at and past the widest row the launch holds (6144), outputs that cut a panel,
+# f32, f16, and groups of two dense types, which take one kernel per matrix
+@pytest.mark.parametrize("hidden,inter,t,vocab,bias", [
+    (20, 8, "ff", 70, False), (255, 131, "ff", 65, True), (256, 260, "hh", 130, True), (516, 1031, "ff", 66, False),
+    (513, 512, "hh", 64, False), (1120, 3040, "hh", 1031, True), (6144, 72, "ff", 40, False), (6148, 72, "ff", 40, True),
+    (6144, 40, "hh", 41, False), (6160, 40, "hh", 41, False), (260, 136, "hf", 70, True), (260, 136, "fh", 70, False)])
+def test_dense_decode_widths(jy, oracle_lib, hidden, inter, t, vocab, bias):
+    a, b = [QM.JY_F32 if c == "f" else QM.JY_F16 for c in t]
+    layer = dict(Wq=a, Wk=a, Wv=b, Wo=a, W1=a, W2=b, W3=b)
+    spec = dict(hidden=hidden, heads=2, kv=1, hd=16, inter=inter, vocab=vocab, theta=10000.0, bias=bias,
+                layers=[layer] * 2, embed=a, lm=b, tied=False)
+    check_forward(jy, oracle_lib, spec, (2, 1, 1))
+    check_generate(jy, oracle_lib, spec)
+
 
 # the prompt GEMMs' tokens per wave (1, 2, 4, 8, 16: by rows and columns), rows that leave a partial
 # wave and workgroup, 64-column tiles cut short, chunks of 256 cut to 32, 64, 96 and 224 (Q8_0),
