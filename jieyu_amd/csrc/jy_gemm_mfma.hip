@@ -645,7 +645,7 @@ static GmChoice gemm_choice(const Q8MfmaDev& W, int m, Epi epi, bool unsplit = f
         int mt, nt;
         float lat, thr;
     };
-    static constexpr Tile tiles[] = {{2, 2, 640.0f, 550.0f}, {1, 2, 400.0f, 305.0f}, {2, 1, 400.0f, 305.0f}, {1, 1, 275.0f, 170.0f}};
+    static constexpr Tile tiles[] = {{2, 2, 640.0f, 550.0f}, {2, 1, 400.0f, 305.0f}, {1, 2, 400.0f, 305.0f}, {1, 1, 275.0f, 170.0f}};
     const int cus = gemm_cus();
     bool all = false;
     const int zmax = unsplit ? 1 : max_slices(W, m, epi, all);
