@@ -13,11 +13,12 @@
 //
 // Layout.  The matrix is kept a second time for these kernels (built when the mode is
 // enabled): for every tile of 16 rows and every block 512 bytes, slot c + 16 g (row c of the
-// tile) holding the 16 bytes k = 16 g .. 16 g + 15 of the block, which one lane of the B
-// operand takes at once; and the block scales as fp32, four blocks of a row together (zero
-// past the last block).  v_mfma_f32_32x32x16_f16 takes 16 k from two lane groups of 8; the
-// kernel gives lane group g of the h-th of a block's two instructions k = 16 g + 8 h .. + 7
-// in both operands: whatever order the instruction gives them, A and B agree on it.
+// tile) holding the 16 bytes k = 8 g .. 8 g + 7 and 16 + 8 g .. 16 + 8 g + 7 of the block, which
+// one lane of the B operand takes at once; and the block scales as fp32, four blocks of a row
+// together (zero past the last block).  v_mfma_f32_32x32x16_f16 takes 16 k from two lane
+// groups of 8; lane group g of the h-th of a block's two instructions has k = 16 h + 8 g .. + 7
+// in both operands, and the two in turn give bit for bit the sum that one
+// v_mfma_f32_16x16x32_f16 over the block gives.
 //
 // Tiling.  A workgroup of 4 waves computes 32 MT rows (tokens) x 128 NT columns (matrix
 // rows), each wave all the rows of its 32 NT columns.  So a wave alone uses its weights and
@@ -51,7 +52,7 @@ typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
 // ---------------------------------------------------------------- the matrix copy
 
 // one thread per (16-row tile t, block b, l): the 8 weights of row 16t + (l % 16),
-// k = 32b + 8(l/16) .. +7, into half (l/16) % 2 of slot (l % 16) + 16 (l/32), from the lane-pair layout (slot r*16 + g of chunk b/8 holds
+// k = 32b + 8(l/16) .. +7, into half l/32 of slot (l % 16) + 16 ((l/16) % 2), from the lane-pair layout (slot r*16 + g of chunk b/8 holds
 // weights 2g, 2g+1 of each of its 8 blocks at bytes 2j, 2j+1); the scales of blocks
 // 4*b4 .. 4*b4+3 of each row by the threads with l < 16 and b % 4 == 0
 __global__ void mfma_repack_kernel(Q8Dev W, Q8MfmaDev M) {
@@ -75,7 +76,7 @@ __global__ void mfma_repack_kernel(Q8Dev W, Q8MfmaDev M) {
         w0 = v[0] | (v[1] << 16);
         w1 = v[2] | (v[3] << 16);
     }
-    uint2* dst = reinterpret_cast<uint2*>(M.q + tb * 512 + (((G >> 1) * 16 + (l % 16)) * 2 + (G & 1)) * 8);
+    uint2* dst = reinterpret_cast<uint2*>(M.q + tb * 512 + (((G & 1) * 16 + (l % 16)) * 2 + (G >> 1)) * 8);
     *dst = make_uint2(w0, w1);
     if (l < 16 && (b & 3) == 0) {
         float4 dv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_mfma_kernel(
     const int tilet = ct * (CC / 16) + wave * 2 * NT;  // the wave's first 16-column tile
     const int nb = W.nb;
     // the workgroup's K slice: blocks [b0, b1), its sums into C's slice y ([z][m][ldc]: the
-    // partials a sum kernel adds); nbz is a multiple of KB
+    // partials a sum kernel adds); in steps of KB blocks from the multiple of KB at or before b0
     const int b0 = (int)blockIdx.y * nbz, b1 = min(nb, b0 + nbz);
     C += (size_t)blockIdx.y * m * ldc;
     const uint32_t base = __builtin_amdgcn_readfirstlane(lds_byte_addr(gsmem));
@@ -390,7 +391,7 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_mfma_kernel(
                 dma_b128(asrc[j] + (size_t)(i & 1) * 8 * K + min(32 * (b + 2 * (i >> 1)) + apc, K - 8),
                          base + buf * ABUF + (uint32_t)((wave * (NA / 4) + j) * 4 + 2 * (i >> 1) + (i & 1)) * 1024);
     };
-    // this lane's column: tile (l & 31) / 16 of a pair, row l % 16 of it; its k: 16 (l / 32) .. +15
+    // this lane's column: tile (l & 31) / 16 of a pair, row l % 16 of it; its k: 8 (l / 32) + 16 h .. +7, h = 0, 1
     const int t0 = min(tilet, W.tiles - 1);
     const __amdgpu_buffer_rsrc_t qr = __builtin_amdgcn_make_buffer_rsrc(
         W.q + (size_t)t0 * nb * 512, 0, (int)min((size_t)(W.tiles - t0) * nb * 512, (size_t)0x7fffffff), 0x00020000);
@@ -407,7 +408,18 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_mfma_kernel(
     };
     auto load_d = [&](int b, float4(&d)[NT]) {
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++) d[nt] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(dr, dof, (nt * 2 * W.nb4 + b / 4) * 256, 0));
+        for (int nt = 0; nt < NT; nt++)
+            d[nt] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(dr, dof, (nt * 2 * W.nb4 + b / 4) * 256, 0));
+    };
+    // the scales of the step at b, zero outside the slice (where they are first used: at the load the
+    // step would wait for it)
+    auto take_d = [&](int b) {
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+            const float4 v = dnxt[nt];
+            dcur[nt] = make_float4(b >= b0 && b < b1 ? v.x : 0.0f, b + 1 >= b0 && b + 1 < b1 ? v.y : 0.0f,
+                                   b + 2 >= b0 && b + 2 < b1 ? v.z : 0.0f, b + 3 >= b0 && b + 3 < b1 ? v.w : 0.0f);
+        }
     };
 
     auto mm = [](h8_t a, h8_t b, f16_t c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); };
@@ -416,7 +428,7 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_mfma_kernel(
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) acc[mt][nt] = f16_t(0.0f);
-    // fragment address: 16-row tile (l & 31) / 16, row l % 16 in it, piece 4 (kb % 2) + 2 (l / 32) + h
+    // fragment address: 16-row tile (l & 31) / 16, row l % 16 in it, piece 4 (kb % 2) + 2 h + l / 32
     const int fr = ((l & 31) >> 4) * 4 * 64 + ((l >> 3) & 1) * 64 + (l & 7) * 8;
     auto block = [&](int buf, int kb) {
         h8_t ah[MT][2], al[MT][2];
@@ -424,7 +436,7 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_mfma_kernel(
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll
             for (int h = 0; h < 2; h++) {
-                const int sl = fr + ((4 * (kb & 1) + 2 * (l >> 5) + h) ^ (l & 7)) + (kb >> 1) * 128;
+                const int sl = fr + ((4 * (kb & 1) + 2 * h + (l >> 5)) ^ (l & 7)) + (kb >> 1) * 128;
                 ah[mt][h] = (&As[buf][0][mt * 2][0][0])[sl];
                 al[mt][h] = (&As[buf][1][mt * 2][0][0])[sl];
             }
@@ -433,8 +445,7 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_mfma_kernel(
             const h8_t bq[2] = {q8_to_h8(q[kb][nt].x, q[kb][nt].y), q8_to_h8(q[kb][nt].z, q[kb][nt].w)};
             const float dv = f4_get(dcur[nt], kb);
             f16_t t[MT];
-            // (high parts first: the low parts ahead of them would save no instruction, and the error
-            // against 64 bits would be 1-3 % larger)
+            // (high parts first; the low parts ahead of them: error against 64 bits 1-3 % larger)
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) t[mt] = mm(ah[mt][0], bq[0], f16_t(0.0f));
 #pragma unroll
@@ -450,15 +461,17 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_mfma_kernel(
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // (a step past the last block: the scales there are zero, the activations repeated, the
-    // weights another tile's or, past the matrix, zero)
+    // (a step's blocks outside the slice: their scales are zero, their activations and weights
+    // the neighbours' or, past the matrix, repeated or zero)
     if (b0 < b1) {
-        issue_a(b0, 0);
+        const int s0 = b0 / KB * KB;
+        issue_a(s0, 0);
 #pragma unroll
-        for (int kb = 0; kb < KB; kb++) load_b(b0, kb);
-        load_d(b0, dcur);
+        for (int kb = 0; kb < KB; kb++) load_b(s0, kb);
+        load_d(s0, dnxt);
+        take_d(s0);
         int buf = 0;
-        for (int b = b0; b < b1; b += KB, buf ^= 1) {
+        for (int b = s0; b < b1; b += KB, buf ^= 1) {
             wait_vm<0>();
             __syncthreads();  // this step's activations are in LDS; the other buffer is read
             if (b + KB < b1) issue_a(b + KB, buf ^ 1);
@@ -469,8 +482,7 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_mfma_kernel(
                 load_b(b + KB, kb);
                 __builtin_amdgcn_sched_barrier(0);
             }
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) dcur[nt] = dnxt[nt];
+            take_d(b + KB);
         }
     }
 
@@ -528,7 +540,7 @@ int mfma_rows_padded(int m) { return (m + GM_TILE - 1) / GM_TILE * GM_TILE; }
 
 // ---------------------------------------------------------------- split over K
 //
-// A grid that leaves CUs idle or with one workgroup, walking a long chain of blocks alone,
+// A small grid that leaves CUs idle, each wave walking a long chain of blocks alone,
 // runs as Z slices of K (gridDim.y), each writing its partial sums [z][m][N] (plain stores),
 // then gemm_ksum_kernel adds the partials in slice order and applies the epilogue: the same
 // result for every run, whatever order the slices finish in.
@@ -615,57 +627,47 @@ static int gemm_cus() {
     return g_gemm_cus;
 }
 
-// The K slices of C = A W^T over m rows.  For outputs of under 16 MiB as many as fill the chip
-// with two 64 x 128 tiles per CU, of at least KSPLIT_MIN_BLOCKS blocks, at most KSPLIT_MAX: the
-// more slices, the fewer additions in a row (4096 x 4096: error against 64 bits 2.1e-7 unsplit,
-// 1.3e-7 with 4), and the partial sums stay within 16 MiB, which callers with a small fixed
-// workspace need.  Larger ones have 1 to KSPLIT_MAX, by time (gemm_choice).  (The SwiGLU
-// epilogue pairs columns and is not split.)
-static int max_slices(const Q8MfmaDev& W, int m, Epi epi, bool& all) {
-    all = (size_t)m * W.rows * sizeof(float) < ((size_t)16 << 20);
-    if (epi == EPI_SWIGLU) return 1;
-    int z = std::min(KSPLIT_MAX, W.nb / KSPLIT_MIN_BLOCKS);
-    if (all) {
-        const int cus = gemm_cus(), tiles = (m + 127) / 128 * 2 * ((W.tiles + 7) / 8);
-        z = tiles >= cus ? 1 : std::min(z, 2 * cus / tiles);
-    }
-    return std::max(1, z);
+// K slices for C = A W^T over m rows: 1 unless 64 x 128 tiles (rows padded to 128) are fewer
+// than the CUs; then up to two such tiles per CU, at most KSPLIT_MAX slices of at least
+// KSPLIT_MIN_BLOCKS blocks, none of them empty.  The count does not follow the tile chosen
+// below: it decides the rounding (4096 x 4096: error against 64 bits 2.1e-7 unsplit, 1.3e-7
+// with 4), and the partial sums' room, which callers with a small fixed workspace count on.
+// (The SwiGLU epilogue pairs columns and is not split.)
+int gemm_q8_mfma_ksplit(const Q8MfmaDev& W, int m, Epi epi) {
+    const int cus = gemm_cus();
+    const long wgs = (long)((m + 127) / 128 * 2) * ((W.tiles + 7) / 8);
+    if (epi == EPI_SWIGLU || wgs >= cus) return 1;
+    const int z = (int)std::min<long>(std::min<long>(KSPLIT_MAX, 2L * cus / std::max(1L, wgs)),
+                                      W.nb / KSPLIT_MIN_BLOCKS);
+    if (z < 2) return 1;
+    const int nbz = (W.nb + z - 1) / z;
+    return (W.nb + nbz - 1) / nbz;
 }
 
-// The tile (32 MT rows x 128 NT columns per workgroup) and the K slices of a launch: the least
-// of nbz blocks x max(lat, thr x the busiest CU's workgroups) ns, where lat is a lone
-// workgroup's time per block and thr the time per block and workgroup of a full CU, plus for
-// slices the partial sums' way through memory.  Measured at 28672 x 4096, 6144 x 4096, 4096 x
-// 4096, 4096 x 14336, 37888 x 3584, 9728 x 896, 1152 x 896 and 896 x 4864, 61 to 1024 rows.
-struct GmChoice {
-    int mt = 1, nt = 1, nbz = 0, z = 1;
+// The tile (32 MT rows x 128 NT columns per workgroup) of a launch with z slices: the least
+// max(lat, thr x the busiest CU's workgroups), where lat is a lone workgroup's ns per block
+// and thr the ns per block and workgroup of a full CU.  Measured at 28672 x 4096, 6144 x
+// 4096, 4096 x 4096, 4096 x 14336, 37888 x 3584, 9728 x 896, 1152 x 896 and 896 x 4864, 61 to
+// 1024 rows.
+struct GmTile {
+    int mt, nt;
+    float lat, thr;
 };
-static GmChoice gemm_choice(const Q8MfmaDev& W, int m, Epi epi, bool unsplit = false) {
-    struct Tile {
-        int mt, nt;
-        float lat, thr;
-    };
-    static constexpr Tile tiles[] = {{2, 2, 640.0f, 550.0f}, {2, 1, 400.0f, 305.0f}, {1, 2, 400.0f, 305.0f}, {1, 1, 275.0f, 170.0f}};
+static GmTile gemm_tile(const Q8MfmaDev& W, int m, int z) {
+    static constexpr GmTile tiles[] = {{2, 2, 640.0f, 550.0f}, {2, 1, 400.0f, 305.0f}, {1, 2, 400.0f, 305.0f}, {1, 1, 275.0f, 170.0f}};
     const int cus = gemm_cus();
-    bool all = false;
-    const int zmax = unsplit ? 1 : max_slices(W, m, epi, all);
-    GmChoice best;
+    GmTile best{};
     float cost = 0.0f;
-    for (const Tile& t : tiles)
-        for (int zi = all ? zmax : 1; zi <= zmax; zi++) {
-            const int nbz = ((W.nb + zi - 1) / zi + GM_KB - 1) / GM_KB * GM_KB, z = (W.nb + nbz - 1) / nbz;
-            const long wgs = (long)((m + 32 * t.mt - 1) / (32 * t.mt)) * ((W.tiles + 8 * t.nt - 1) / (8 * t.nt)) * z;
-            float c = (float)nbz * std::max(t.lat, t.thr * (float)((wgs + cus - 1) / cus));
-            if (z > 1) c += 1500.0f + (float)z * (float)m * (float)W.rows * (8.0f / 4000.0f);
-            if (!best.nbz || c < cost) {
-                cost = c;
-                best.mt = t.mt, best.nt = t.nt, best.nbz = nbz, best.z = z;
-            }
+    for (const GmTile& t : tiles) {
+        const long wgs = (long)((m + 32 * t.mt - 1) / (32 * t.mt)) * ((W.tiles + 8 * t.nt - 1) / (8 * t.nt)) * z;
+        const float c = std::max(t.lat, t.thr * (float)((wgs + cus - 1) / cus));
+        if (!best.mt || c < cost) {
+            cost = c;
+            best = t;
         }
+    }
     return best;
 }
-
-int gemm_q8_mfma_ksplit(const Q8MfmaDev& W, int m, Epi epi) { return gemm_choice(W, m, epi).z; }
 
 size_t gemm_q8_mfma_kpart_floats(const Q8MfmaDev& W, int m, Epi epi) {
     const int z = gemm_q8_mfma_ksplit(W, m, epi);
@@ -675,18 +677,19 @@ size_t gemm_q8_mfma_kpart_floats(const Q8MfmaDev& W, int m, Epi epi) {
 int launch_gemm_q8_mfma(const Q8MfmaDev& W, int m, const _Float16* hi, const _Float16* lo, const float* unscale,
                         float* C, int ldc, const float* aux, Epi epi, hipStream_t st, float* kpart, size_t kpart_n,
                         bool defer) {
-    GmChoice g = gemm_choice(W, m, epi);
-    if (g.z > 1 && (!kpart || (size_t)g.z * m * W.rows > kpart_n)) g = gemm_choice(W, m, epi, true);
-    const int Z = g.z;
+    int Z = gemm_q8_mfma_ksplit(W, m, epi);
+    if (Z > 1 && (!kpart || (size_t)Z * m * W.rows > kpart_n)) Z = 1;
+    const GmTile g = gemm_tile(W, m, Z);
+    const int nbz = (W.nb + Z - 1) / Z;
     auto run = [&](float* out, int ld, const float* ax, Epi e) {
         if (g.mt == 2 && g.nt == 2)
-            gemm_launch<2, 2>(W, m, hi, lo, unscale, out, ld, ax, e, st, g.nbz);
+            gemm_launch<2, 2>(W, m, hi, lo, unscale, out, ld, ax, e, st, nbz);
         else if (g.mt == 2)
-            gemm_launch<2, 1>(W, m, hi, lo, unscale, out, ld, ax, e, st, g.nbz);
+            gemm_launch<2, 1>(W, m, hi, lo, unscale, out, ld, ax, e, st, nbz);
         else if (g.nt == 2)
-            gemm_launch<1, 2>(W, m, hi, lo, unscale, out, ld, ax, e, st, g.nbz);
+            gemm_launch<1, 2>(W, m, hi, lo, unscale, out, ld, ax, e, st, nbz);
         else
-            gemm_launch<1, 1>(W, m, hi, lo, unscale, out, ld, ax, e, st, g.nbz);
+            gemm_launch<1, 1>(W, m, hi, lo, unscale, out, ld, ax, e, st, nbz);
     };
     if (Z < 2) {
         run(C, ldc, aux, epi);

@@ -146,7 +146,10 @@ hipError_t HostStage::to_device(void* dst, const void* src, size_t n, hipStream_
         // a slot is free again once the copy of the chunk it held has run
         while (opened < nch && opened - SLOTS < sent) {
             e = hipEventQuery(ev_[opened % SLOTS]);
-            if (e == hipErrorNotReady) break;
+            if (e == hipErrorNotReady) {
+                (void)hipGetLastError();  // (an answer, not an error to be found after the next launch)
+                break;
+            }
             if (e != hipSuccess) return e;
             team.open(++opened);
         }
@@ -187,7 +190,10 @@ hipError_t HostStage::to_host(void* dst, size_t rows, size_t row_bytes, hipStrea
     while (copied < nch) {
         while (opened < sent) {
             e = hipEventQuery(ev_[opened % SLOTS]);
-            if (e == hipErrorNotReady) break;
+            if (e == hipErrorNotReady) {
+                (void)hipGetLastError();
+                break;
+            }
             if (e != hipSuccess) return e;
             team.open(++opened);
         }
