@@ -159,7 +159,7 @@ def isolated_prompt_gemm(jy, d, n, iters=8):
     us = min(m.gemm_time(A, iters) for _ in range(3))
     m.close()
     useful = 2.0 * n * rows * cols / (us * 1e-6) / 1e12
-    return {"bound": "mfma", "kernel": "gemm_q8_mfma2_kernel (gate/up, %d x %d, %d rows)" % (rows, cols, n),
+    return {"bound": "mfma", "kernel": "gemm_q8_mfma_kernel (gate/up, %d x %d, %d rows)" % (rows, cols, n),
             "us": round(us, 1), "gemm_tflops": round(useful, 1), "mfma_executed_tflops": round(2 * useful, 1),
             "peak_tflops": F16_MFMA_PEAK_TFLOPS, "mfma_frac": round(2 * useful / F16_MFMA_PEAK_TFLOPS, 4)}
 
