@@ -645,22 +645,25 @@ int gemm_q8_mfma_ksplit(const Q8MfmaDev& W, int m, Epi epi) {
 }
 
 // The tile (32 MT rows x 128 NT columns per workgroup) of a launch with z slices: the least
-// max(lat, thr x the busiest CU's workgroups), where lat is a lone workgroup's ns per block
-// and thr the ns per block and workgroup of a full CU.  Measured at 28672 x 4096, 6144 x
+// max(lat, thr x the busiest CU's workgroups + off), where lat is a lone workgroup's ns per
+// block and thr the ns per block and workgroup of a full CU (32 x 256 gains on 64 x 128 from
+// three workgroups: 6144 x 4096 at 1024 rows 120 us against 133; at two, 4096 x 14336, 285
+// against 272).  Measured at 28672 x 4096, 6144 x
 // 4096, 4096 x 4096, 4096 x 14336, 37888 x 3584, 9728 x 896, 1152 x 896 and 896 x 4864, 61 to
 // 1024 rows.
 struct GmTile {
     int mt, nt;
-    float lat, thr;
+    float lat, thr, off;
 };
 static GmTile gemm_tile(const Q8MfmaDev& W, int m, int z) {
-    static constexpr GmTile tiles[] = {{2, 2, 640.0f, 550.0f}, {2, 1, 400.0f, 305.0f}, {1, 2, 400.0f, 305.0f}, {1, 1, 275.0f, 170.0f}};
+    static constexpr GmTile tiles[] = {{2, 2, 640.0f, 550.0f, 0.0f}, {2, 1, 400.0f, 312.0f, 0.0f},
+                                       {1, 2, 400.0f, 290.0f, 60.0f}, {1, 1, 275.0f, 170.0f, 0.0f}};
     const int cus = gemm_cus();
     GmTile best{};
     float cost = 0.0f;
     for (const GmTile& t : tiles) {
         const long wgs = (long)((m + 32 * t.mt - 1) / (32 * t.mt)) * ((W.tiles + 8 * t.nt - 1) / (8 * t.nt)) * z;
-        const float c = std::max(t.lat, t.thr * (float)((wgs + cus - 1) / cus));
+        const float c = std::max(t.lat, t.thr * (float)((wgs + cus - 1) / cus) + t.off);
         if (!best.mt || c < cost) {
             cost = c;
             best = t;
