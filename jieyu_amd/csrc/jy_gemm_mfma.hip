@@ -39,6 +39,7 @@
 #include <algorithm>
 #include <cstddef>
 
+#include "jy_gemm_offsets.h"
 #include "jy_layout.h"
 #include "jy_mfma.h"
 
@@ -391,25 +392,30 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_mfma_kernel(
                 dma_b128(asrc[j] + (size_t)(i & 1) * 8 * K + min(32 * (b + 2 * (i >> 1)) + apc, K - 8),
                          base + buf * ABUF + (uint32_t)((wave * (NA / 4) + j) * 4 + 2 * (i >> 1) + (i & 1)) * 1024);
     };
-    // this lane's column: tile (l & 31) / 16 of a pair, row l % 16 of it; its k: 8 (l / 32) + 16 h .. +7, h = 0, 1
-    const int t0 = min(tilet, W.tiles - 1);
+    // this lane's column: tile (l & 31) / 16 of a pair, row l % 16 of it; its k: 8 (l / 32) + 16 h .. +7, h = 0, 1.
+    // Every load is inside the copy by its own offsets (jy_gemm_offsets.h)
+    const int t0 = gm_base_tile(tilet, W.tiles);
     const __amdgpu_buffer_rsrc_t qr = __builtin_amdgcn_make_buffer_rsrc(
         W.q + (size_t)t0 * nb * 512, 0, (int)min((size_t)(W.tiles - t0) * nb * 512, (size_t)0x7fffffff), 0x00020000);
     const __amdgpu_buffer_rsrc_t dr = __builtin_amdgcn_make_buffer_rsrc(
         W.d + (size_t)t0 * W.nb4 * 64, 0, (int)min((size_t)(W.tiles - t0) * W.nb4 * 256, (size_t)0x7fffffff), 0x00020000);
-    const int qo = ((l & 31) >> 4) * nb * 512 + (l & 15) * 16 + 256 * (l >> 5);
-    const int dof = ((l & 31) >> 4) * W.nb4 * 256 + (l & 15) * 16;
+    int qo[NT], dof[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+        qo[nt] = gm_q_lane(tilet, nt, l, W.tiles, nb);
+        dof[nt] = gm_d_lane(tilet, nt, l, W.tiles, W.nb4);
+    }
     uint4 q[KB][NT];
     float4 dcur[NT], dnxt[NT];
     auto load_b = [&](int b, int kb) {
 #pragma unroll
         for (int nt = 0; nt < NT; nt++)
-            q[kb][nt] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(qr, qo, (nt * 2 * nb + b + kb) * 512, 0));
+            q[kb][nt] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(qr, qo[nt], gm_q_block(b + kb, nb), 0));
     };
     auto load_d = [&](int b, float4(&d)[NT]) {
 #pragma unroll
         for (int nt = 0; nt < NT; nt++)
-            d[nt] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(dr, dof, (nt * 2 * W.nb4 + b / 4) * 256, 0));
+            d[nt] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(dr, dof[nt], gm_d_block(b, W.nb4), 0));
     };
     // the scales of the step at b, zero outside the slice (where they are first used: at the load the
     // step would wait for it)
@@ -462,7 +468,7 @@ __global__ __launch_bounds__(256, 2) void gemm_q8_mfma_kernel(
         }
     };
     // (a step's blocks outside the slice: their scales are zero, their activations and weights
-    // the neighbours' or, past the matrix, repeated or zero)
+    // the neighbours' or, past the matrix, repeated)
     if (b0 < b1) {
         const int s0 = b0 / KB * KB;
         issue_a(s0, 0);
