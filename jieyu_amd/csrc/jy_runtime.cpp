@@ -1596,22 +1596,23 @@ int generate_impl(jyhip_model* m, jyhip_kv* kv_in, const int* prompt, int plen, 
 
 
 // a forward call's rows into w.X, and the final RMSNorm (forward.h:86-94) of w.X's rows to the
-// caller, the stream waited for
-void rows_in(jyhip_model* m, Workspace& w, const float* X, int seq) {
+// caller, the stream waited for; `threads`: many rows may be copied by helper threads
+void rows_in(jyhip_model* m, Workspace& w, const float* X, int seq, bool threads) {
     const size_t n = sizeof(float) * seq * m->H;
     if (m->stage.ready())
-        CK(m->stage.to_device(w.X, X, n, m->stream));
+        CK(m->stage.to_device(w.X, X, n, m->stream, threads));
     else
         CK(hipMemcpyAsync(w.X, X, n, hipMemcpyHostToDevice, m->stream));
 }
 
-void rows_out(jyhip_model* m, Workspace& w, float* out, int seq) {
+void rows_out(jyhip_model* m, Workspace& w, float* out, int seq, bool threads) {
     hipStream_t st = m->stream;
     const size_t row = sizeof(float) * m->H;
-    if (m->stage.ready() && row <= HostStage::SLOT) {  // the norm writes the pinned ring itself
-        CK(m->stage.to_host(out, seq, row, st, [&](size_t r0, size_t n, void* p) {
+    if (m->stage.ready()) {  // the norm writes the pinned ring itself
+        const auto norm = [&](size_t r0, size_t n, void* p) {
             launch_rmsnorm(w.X + r0 * m->H, static_cast<float*>(p), m->final_rms, m->H, (int)n, st);
-        }));
+        };
+        CK(m->stage.to_host(out, seq, row, st, norm, threads));
         return;
     }
     launch_rmsnorm(w.X, w.xn, m->final_rms, m->H, seq, st);
@@ -1634,9 +1635,9 @@ int forward_impl(jyhip_model* m, jyhip_kv* kv, const float* X, float* out, int s
     ensure_scores(m, scores_need(m, seq, max_keys));
     ensure_part(m, part_need(m, max_keys));
     Workspace& w = m->ws;
-    rows_in(m, w, X, seq);
+    rows_in(m, w, X, seq, true);
     run_layers(m, w, kv->dev, seq, start_pos, nullptr, layer_out, max_keys);
-    rows_out(m, w, out, seq);
+    rows_out(m, w, out, seq, true);
     check_persist(m);
     kv->current_len = start_pos + seq;
     return 0;
@@ -1683,7 +1684,7 @@ Workspace ws_view(const jyhip_model* m, int seq, int max_keys, size_t scores_n, 
 }
 
 // forward_cached over the GPU's static scratch: the checks and steps of forward_impl
-// (layer outputs aside) with no device allocation
+// (layer outputs aside) with no device allocation, and none on the host for its rows
 int forward_noalloc(jyhip_model* m, jyhip_kv* kv, float* X, int seq, int start_pos) {
     if (!kv || !X) fail("forward: NULL kv or X");
     if (kv->dev.num_layers < m->L || kv->dev.nkv != m->nkv || kv->dev.hd != m->hd)
@@ -1705,9 +1706,9 @@ int forward_noalloc(jyhip_model* m, jyhip_kv* kv, float* X, int seq, int start_p
     // the allocating path starts from zeroed buffers; so does this one, whatever an
     // earlier call left in the shared array
     launch_zero_fill(base, need, m->stream);
-    rows_in(m, w, X, seq);
+    rows_in(m, w, X, seq, false);
     run_layers(m, w, kv->dev, seq, start_pos, nullptr, nullptr, max_keys);
-    rows_out(m, w, X, seq);
+    rows_out(m, w, X, seq, false);
     check_persist(m);
     kv->current_len = start_pos + seq;
     return 0;

@@ -6,7 +6,6 @@
 #include <cstring>
 #include <system_error>
 #include <thread>
-#include <vector>
 
 namespace jy {
 
@@ -32,24 +31,25 @@ void launch_copy(const void* s, void* d, size_t bytes, hipStream_t st) {
 }
 
 // The pieces of a transfer's chunks, claimed in order by whoever is free; a piece may be
-// claimed once its chunk is opened.
+// claimed once its chunk is opened.  Nothing but help() allocates.
+template <class Copy>  // copy(chunk, offset in it, bytes)
 class Team {
   public:
     static constexpr size_t PIECE = (size_t)64 << 10;
 
-    // copy(chunk, offset in it, bytes)
-    Team(size_t chunk, size_t last, size_t nch, std::function<void(size_t, size_t, size_t)> copy)
+    Team(size_t chunk, size_t last, size_t nch, const Copy& copy)
         : chunk_(chunk), last_(last), nch_(nch), per_((chunk + PIECE - 1) / PIECE),
-          total_((nch - 1) * per_ + (last + PIECE - 1) / PIECE), done_(nch), copy_(std::move(copy)) {}
+          total_((nch - 1) * per_ + (last + PIECE - 1) / PIECE), copy_(copy) {}
     ~Team() {
         next_.store(total_);  // (after an error: no more claims)
-        for (std::thread& t : threads_) t.join();
+        for (std::thread& t : threads_)
+            if (t.joinable()) t.join();
     }
-    void help(int n) {
-        n = std::min(n, (int)std::thread::hardware_concurrency() - 1);
+    void help() {
+        const int n = std::min(HostStage::HELPERS, (int)std::thread::hardware_concurrency() - 1);
         try {
             for (int i = 0; i < n; i++)
-                threads_.emplace_back([this] {
+                threads_[i] = std::thread([this] {
                     for (int spin = 0; next_.load(std::memory_order_relaxed) < total_;) {
                         if (work())
                             spin = 0;
@@ -60,7 +60,13 @@ class Team {
         } catch (const std::system_error&) {  // no thread to be had: the caller copies alone
         }
     }
-    void open(size_t chunks) { limit_.store(std::min(chunks * per_, total_), std::memory_order_release); }
+    // (the caller's thread) the next chunk, whose slot's last chunk is complete
+    void open_next() {
+        done_[opened_ % HostStage::SLOTS].store(0, std::memory_order_relaxed);
+        opened_++;
+        limit_.store(std::min(opened_ * per_, total_), std::memory_order_release);
+    }
+    size_t opened() const { return opened_; }
     // one piece, if an opened one is left
     bool work() {
         size_t i = next_.load(std::memory_order_relaxed);
@@ -69,20 +75,22 @@ class Team {
         } while (!next_.compare_exchange_weak(i, i + 1));
         const size_t c = i / per_, off = (i - c * per_) * PIECE;
         copy_(c, off, std::min(PIECE, (c + 1 == nch_ ? last_ : chunk_) - off));
-        done_[c].fetch_add(1, std::memory_order_release);
+        done_[c % HostStage::SLOTS].fetch_add(1, std::memory_order_release);
         return true;
     }
+    // (the caller's thread) whether chunk c, one of the last SLOTS opened or not opened yet, is copied
     bool complete(size_t c) const {
         const size_t n = ((c + 1 == nch_ ? last_ : chunk_) + PIECE - 1) / PIECE;
-        return done_[c].load(std::memory_order_acquire) == n;
+        return c < opened_ && done_[c % HostStage::SLOTS].load(std::memory_order_acquire) == n;
     }
 
   private:
     const size_t chunk_, last_, nch_, per_, total_;
+    size_t opened_ = 0;
     std::atomic<size_t> next_{0}, limit_{0};
-    std::vector<std::atomic<unsigned>> done_;
-    std::function<void(size_t, size_t, size_t)> copy_;
-    std::vector<std::thread> threads_;
+    std::atomic<unsigned> done_[HostStage::SLOTS] = {};  // pieces copied of the chunk in each slot
+    const Copy& copy_;
+    std::thread threads_[HostStage::HELPERS];
 };
 
 }  // namespace
@@ -116,7 +124,7 @@ hipError_t HostStage::idle(hipStream_t st) {
     return e;
 }
 
-hipError_t HostStage::to_device(void* dst, const void* src, size_t n, hipStream_t st) {
+hipError_t HostStage::to_device(void* dst, const void* src, size_t n, hipStream_t st, bool threads) {
     hipError_t e = idle(st);
     if (e != hipSuccess || n == 0) return e;
     busy_ = true;  // (until to_host has waited for the stream)
@@ -128,40 +136,42 @@ hipError_t HostStage::to_device(void* dst, const void* src, size_t n, hipStream_
         launch_copy(ring_, d, n, st);
         return hipGetLastError();
     }
-    Team team(SLOT, last, nch, [&](size_t c, size_t off, size_t len) {
+    auto copy = [&](size_t c, size_t off, size_t len) {
         memcpy(ring_ + (c % SLOTS) * SLOT + off, s + c * SLOT + off, len);
-    });
-    size_t opened = std::min<size_t>(nch, SLOTS), sent = 0;
-    team.open(opened);
-    if (n >= MT_BYTES) team.help(HELPERS);
+    };
+    Team<decltype(copy)> team(SLOT, last, nch, copy);
+    while (team.opened() < std::min<size_t>(nch, SLOTS)) team.open_next();
+    if (threads && n >= MT_BYTES) team.help();
+    size_t sent = 0;
     while (sent < nch) {
         if (team.complete(sent)) {
             launch_copy(ring_ + (sent % SLOTS) * SLOT, d + sent * SLOT, sent + 1 == nch ? last : SLOT, st);
             if ((e = hipGetLastError()) != hipSuccess) return e;
             if ((e = hipEventRecord(ev_[sent % SLOTS], st)) != hipSuccess) return e;
             sent++;
-        } else if (!team.work() && opened == nch) {
+        } else if (!team.work() && team.opened() == nch) {
             std::this_thread::yield();
         }
         // a slot is free again once the copy of the chunk it held has run
-        while (opened < nch && opened - SLOTS < sent) {
-            e = hipEventQuery(ev_[opened % SLOTS]);
+        while (team.opened() < nch && team.opened() - SLOTS < sent) {
+            e = hipEventQuery(ev_[team.opened() % SLOTS]);
             if (e == hipErrorNotReady) {
                 (void)hipGetLastError();  // (an answer, not an error to be found after the next launch)
                 break;
             }
             if (e != hipSuccess) return e;
-            team.open(++opened);
+            team.open_next();
         }
     }
     return hipSuccess;
 }
 
-hipError_t HostStage::to_host(void* dst, size_t rows, size_t row_bytes, hipStream_t st,
-                              const std::function<void(size_t, size_t, void*)>& produce) {
+hipError_t HostStage::to_host(void* dst, size_t rows, size_t row_bytes, hipStream_t st, RowProducer produce,
+                              bool threads) {
+    if (row_bytes > SLOT) return hipErrorInvalidValue;
     hipError_t e = hipSuccess;
     busy_ = true;
-    const size_t rpc = std::max<size_t>(1, SLOT / row_bytes), nch = (rows + rpc - 1) / rpc;
+    const size_t rpc = SLOT / row_bytes, nch = (rows + rpc - 1) / rpc;
     const size_t chunk = rpc * row_bytes, last = rows * row_bytes - (nch - 1) * chunk;
     auto* d = static_cast<unsigned char*>(dst);
     // (the slots' copies to the GPU are ahead of the producers on the stream)
@@ -172,10 +182,11 @@ hipError_t HostStage::to_host(void* dst, size_t rows, size_t row_bytes, hipStrea
         memcpy(d, ring_, rows * row_bytes);
         return hipSuccess;
     }
-    Team team(chunk, last, nch, [&](size_t c, size_t off, size_t len) {
+    auto copy = [&](size_t c, size_t off, size_t len) {
         memcpy(d + c * chunk + off, ring_ + (c % SLOTS) * SLOT + off, len);
-    });
-    size_t sent = 0, opened = 0, copied = 0;
+    };
+    Team<decltype(copy)> team(chunk, last, nch, copy);
+    size_t sent = 0, copied = 0;
     auto send = [&]() {
         produce(sent * rpc, std::min(rpc, rows - sent * rpc), ring_ + (sent % SLOTS) * SLOT);
         if ((e = hipGetLastError()) == hipSuccess) e = hipEventRecord(ev_[sent % SLOTS], st);
@@ -185,17 +196,17 @@ hipError_t HostStage::to_host(void* dst, size_t rows, size_t row_bytes, hipStrea
     while (sent < std::min<size_t>(nch, SLOTS))
         if (!send()) return e;
     if ((e = hipEventSynchronize(ev_[0])) != hipSuccess) return e;  // (the call's work before it)
-    team.open(opened = 1);
-    if (rows * row_bytes >= MT_BYTES) team.help(HELPERS);
+    team.open_next();
+    if (threads && rows * row_bytes >= MT_BYTES) team.help();
     while (copied < nch) {
-        while (opened < sent) {
-            e = hipEventQuery(ev_[opened % SLOTS]);
+        while (team.opened() < sent) {
+            e = hipEventQuery(ev_[team.opened() % SLOTS]);
             if (e == hipErrorNotReady) {
                 (void)hipGetLastError();
                 break;
             }
             if (e != hipSuccess) return e;
-            team.open(++opened);
+            team.open_next();
         }
         if (team.complete(copied)) {
             copied++;

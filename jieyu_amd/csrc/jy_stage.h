@@ -5,14 +5,30 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
-#include <functional>
 
 namespace jy {
 
+// produce(first row, rows, where) of to_host: a callable by reference, for the length of the call
+// (std::function may allocate)
+class RowProducer {
+  public:
+    template <class F>
+    RowProducer(const F& f)
+        : ctx_(&f), call_([](const void* c, size_t r0, size_t n, void* where) {
+              (*static_cast<const F*>(c))(r0, n, where);
+          }) {}
+    void operator()(size_t r0, size_t n, void* where) const { call_(ctx_, r0, n, where); }
+
+  private:
+    const void* ctx_;
+    void (*call_)(const void*, size_t, size_t, void*);
+};
+
 // One ring per model: SLOTS slots of SLOT bytes.  The GPU side of a transfer is a kernel that
 // reads or writes a slot (to_device's copy; to_host's producer, which may be the kernel that
-// computes the rows), the host side memcpy by the calling thread and, from MT_BYTES on, up to
-// HELPERS threads that live for the transfer; the two overlap chunk by chunk.
+// computes the rows), the host side memcpy by the calling thread and, with `threads` and from
+// MT_BYTES on, up to HELPERS threads that live for the transfer; the two overlap chunk by chunk.
+// Without `threads` a transfer allocates nothing.
 // The runtime's own copy of pageable memory stages it on one thread, copy after copy: 1024 x
 // 4096 floats to the GPU and back took about 2.4 ms of a call, against 0.6 for the bytes over
 // the bus.
@@ -27,11 +43,10 @@ class HostStage {
     bool ready() const { return ring_ != nullptr; }
 
     // dst (device) = src, n bytes (a multiple of 4), in order on st; src may be reused at once
-    hipError_t to_device(void* dst, const void* src, size_t n, hipStream_t st);
+    hipError_t to_device(void* dst, const void* src, size_t n, hipStream_t st, bool threads);
     // dst = `rows` rows of row_bytes (a multiple of 4, at most SLOT), which produce(first row,
     // rows, where) writes by kernels it enqueues on st; all of it has arrived, and st is idle, on return
-    hipError_t to_host(void* dst, size_t rows, size_t row_bytes, hipStream_t st,
-                       const std::function<void(size_t, size_t, void*)>& produce);
+    hipError_t to_host(void* dst, size_t rows, size_t row_bytes, hipStream_t st, RowProducer produce, bool threads);
 
   private:
     hipError_t idle(hipStream_t st);

@@ -43,3 +43,25 @@ def test_rows_round_trip(jy, oracle_lib, hidden, rows):
     kv.close()
     g.close()
     s.close()
+
+
+# under and over a slot, and over the helpers' 1 MiB: the entry point that allocates nothing copies
+# on the calling thread alone
+@pytest.mark.parametrize("rows", [3, 513, 1025])
+def test_noalloc_rows(jy, oracle_lib, rows):
+    from jieyu_amd.model import Synth, synth_config
+    hidden = 256
+    print(f"[gpu-case] noalloc stage {hidden} x {rows}", flush=True)
+    s = Synth(oracle_lib, synth_config("tiny-f32", num_layers=1, hidden=hidden, num_heads=1, num_kv_heads=1, head_dim=16,
+                                       intermediate=16, vocab_size=16))
+    g = jy.GpuModel(s.desc, rows)
+    kv = g.kv()
+    X = np.random.default_rng(rows).standard_normal((rows, hidden)).astype(np.float32)
+    first = g.forward_cached_noalloc(kv, X, 0)
+    want = g.forward_cached(kv, X, 0)
+    again = g.forward_cached_noalloc(kv, X, 0)
+    for got in (first, again):
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    kv.close()
+    g.close()
+    s.close()

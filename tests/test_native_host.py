@@ -36,3 +36,18 @@ def test_prompt_gemm_weight_loads_stay_inside(gemm_offsets, nt, slices):
     for rows in (1, 16, 17, 32, 77, 130, 896, 1152, 4112, 4608):
         for cols in (32, 64, 96, 128, 160, 896, 4864, 14336):
             assert gemm_offsets(rows, cols, nt, slices) == 0, (rows, cols)
+
+
+@pytest.fixture(scope="module")
+def stage(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("native") / "stage"
+    compile_native(exe, "-pthread", "-I", os.path.join(NATIVE, "hip_stub"), os.path.join(NATIVE, "stage.cpp"),
+                   os.path.join(CSRC, "jy_stage.cpp"))
+    return exe
+
+
+# no_host_allocation: jyhip_forward_cached_noalloc's transfers, of any size
+@pytest.mark.parametrize("case", ["round_trip", "no_host_allocation", "after_an_error"])
+def test_pinned_ring(stage, case):
+    r = subprocess.run([str(stage), case], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
