@@ -163,7 +163,7 @@ struct jyhip_model {
     size_t pk_flag_bytes = 0;
     int* pk_err = nullptr;         // set by the kernel when a barrier wait gave up
     size_t pk_lds = 0;
-    HostStage stage;  // forward calls' rows in and out (where it has no ring: plain copies)
+    HostStage stage;  // forward calls' rows in and out (while it has no ring: plain copies)
     std::vector<void*> owned;
 };
 
@@ -677,7 +677,6 @@ void upload(jyhip_model* m, const jy_model_desc* d, int max_seq, int wtype) {
     m->max_seq = max_seq;
     m->theta = d->rope_theta;
     CK(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
-    (void)m->stage.init();
 
     std::vector<float> c, s;
     rope_table(max_seq, m->hd, m->theta, c, s);
@@ -1596,23 +1595,24 @@ int generate_impl(jyhip_model* m, jyhip_kv* kv_in, const int* prompt, int plen, 
 
 
 // a forward call's rows into w.X, and the final RMSNorm (forward.h:86-94) of w.X's rows to the
-// caller, the stream waited for; `threads`: many rows may be copied by helper threads
-void rows_in(jyhip_model* m, Workspace& w, const float* X, int seq, bool threads) {
+// caller, the stream waited for.  `alloc`: the call may allocate on the host (the pinned ring, made
+// by the model's first such call, and helper threads for many rows)
+void rows_in(jyhip_model* m, Workspace& w, const float* X, int seq, bool alloc) {
     const size_t n = sizeof(float) * seq * m->H;
-    if (m->stage.ready())
-        CK(m->stage.to_device(w.X, X, n, m->stream, threads));
+    if (m->stage.ready(alloc))
+        CK(m->stage.to_device(w.X, X, n, m->stream, alloc));
     else
         CK(hipMemcpyAsync(w.X, X, n, hipMemcpyHostToDevice, m->stream));
 }
 
-void rows_out(jyhip_model* m, Workspace& w, float* out, int seq, bool threads) {
+void rows_out(jyhip_model* m, Workspace& w, float* out, int seq, bool alloc) {
     hipStream_t st = m->stream;
     const size_t row = sizeof(float) * m->H;
-    if (m->stage.ready()) {  // the norm writes the pinned ring itself
+    if (m->stage.ready(alloc)) {  // the norm writes the pinned ring itself
         const auto norm = [&](size_t r0, size_t n, void* p) {
             launch_rmsnorm(w.X + r0 * m->H, static_cast<float*>(p), m->final_rms, m->H, (int)n, st);
         };
-        CK(m->stage.to_host(out, seq, row, st, norm, threads));
+        CK(m->stage.to_host(out, seq, row, st, norm, alloc));
         return;
     }
     launch_rmsnorm(w.X, w.xn, m->final_rms, m->H, seq, st);

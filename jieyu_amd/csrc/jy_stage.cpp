@@ -95,6 +95,14 @@ class Team {
 
 }  // namespace
 
+bool HostStage::ready(bool create) {
+    if (!ring_ && create && !tried_) {
+        tried_ = true;
+        return init();
+    }
+    return ring_ != nullptr;
+}
+
 bool HostStage::init() {
     void* p = nullptr;
     bool ok = hipHostMalloc(&p, SLOT * SLOTS, hipHostMallocDefault) == hipSuccess;

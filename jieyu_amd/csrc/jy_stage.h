@@ -37,10 +37,12 @@ class HostStage {
     static constexpr size_t SLOT = (size_t)512 << 10, MT_BYTES = (size_t)1 << 20;
     static constexpr int SLOTS = 8, HELPERS = 3;
 
-    // allocates; false (and no ring: the calls below may not be made) where it cannot
-    bool init();
+    // whether there is a ring (else the calls below may not be made).  With `create` the first
+    // call makes it, and where it cannot no later one tries: a model that never takes rows from
+    // the host (generation, sessions) holds no pinned memory.  (About 50 us of that call; the first
+    // touch of its pages, ~0.4 us per KiB used, falls on the calls that use them either way.)
+    bool ready(bool create);
     void release();
-    bool ready() const { return ring_ != nullptr; }
 
     // dst (device) = src, n bytes (a multiple of 4), in order on st; src may be reused at once
     hipError_t to_device(void* dst, const void* src, size_t n, hipStream_t st, bool threads);
@@ -49,9 +51,11 @@ class HostStage {
     hipError_t to_host(void* dst, size_t rows, size_t row_bytes, hipStream_t st, RowProducer produce, bool threads);
 
   private:
+    bool init();
     hipError_t idle(hipStream_t st);
     unsigned char* ring_ = nullptr;
     hipEvent_t ev_[SLOTS] = {};
+    bool tried_ = false;
     bool busy_ = false;  // a transfer was begun and not seen to its end
 };
 

@@ -40,7 +40,7 @@ struct Op {
 };
 inline Op g_ops[4096];
 inline size_t g_put = 0, g_done = 0;
-inline int g_host_allocs = 0, g_host_frees = 0, g_events = 0;
+inline int g_host_allocs = 0, g_host_frees = 0, g_events = 0, g_live_events = 0;
 inline int g_fail_host_malloc = 0, g_fail_event_at = 0, g_fail_record_in = 0;  // (0: never)
 
 inline void run_to(size_t n) {
@@ -88,10 +88,12 @@ inline hipError_t hipHostFree(void* p) {
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
     if (hip_stub::g_fail_event_at && ++hip_stub::g_events == hip_stub::g_fail_event_at) return hipErrorOutOfMemory;
     *e = new StubEvent;
+    hip_stub::g_live_events++;
     return hipSuccess;
 }
 inline hipError_t hipEventDestroy(hipEvent_t e) {
     delete e;
+    hip_stub::g_live_events--;
     return hipSuccess;
 }
 inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {

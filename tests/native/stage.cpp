@@ -61,7 +61,28 @@ static const size_t SIZES[][2] = {{1, 1},      {3, 5},      {1, 4096},    {33, 4
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     HostStage s;
-    CHECK(s.init());
+    if (!strcmp(what, "made_when_needed")) {
+        CHECK(!s.ready(false) && hip_stub::g_host_allocs == 0);
+        CHECK(s.ready(true) && s.ready(false) && s.ready(true) && hip_stub::g_host_allocs == 1);
+        s.release();
+        CHECK(hip_stub::g_host_frees == 1);
+        // no pinned memory, or no k-th event: no ring, nothing left behind, no second try
+        for (int k = 0; k <= HostStage::SLOTS; k++) {
+            HostStage f;
+            hip_stub::g_fail_host_malloc = k == 0;
+            hip_stub::g_fail_event_at = k;
+            hip_stub::g_events = 0;
+            const int before = hip_stub::g_host_allocs;
+            CHECK(!f.ready(true));
+            hip_stub::g_fail_host_malloc = hip_stub::g_fail_event_at = 0;
+            CHECK(!f.ready(true) && !f.ready(false));
+            CHECK(hip_stub::g_host_allocs == before + (k != 0) && hip_stub::g_host_allocs == hip_stub::g_host_frees);
+            CHECK(hip_stub::g_live_events == 0);
+            f.release();
+        }
+        return 0;
+    }
+    CHECK(s.ready(true));
     if (!strcmp(what, "round_trip")) {
         for (int pass = 0; pass < 3; pass++)
             for (const auto& z : SIZES) round_trip(s, z[0], z[1], pass != 1, 17 * pass + 1);
@@ -100,6 +121,6 @@ int main(int argc, char** argv) {
     }
     hipStreamSynchronize(nullptr);
     s.release();
-    CHECK(hip_stub::g_host_allocs == hip_stub::g_host_frees);
+    CHECK(hip_stub::g_host_allocs == hip_stub::g_host_frees && hip_stub::g_live_events == 0);
     return 0;
 }

@@ -47,7 +47,7 @@ def stage(tmp_path_factory):
 
 
 # no_host_allocation: jyhip_forward_cached_noalloc's transfers, of any size
-@pytest.mark.parametrize("case", ["round_trip", "no_host_allocation", "after_an_error"])
+@pytest.mark.parametrize("case", ["made_when_needed", "round_trip", "no_host_allocation", "after_an_error"])
 def test_pinned_ring(stage, case):
     r = subprocess.run([str(stage), case], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
