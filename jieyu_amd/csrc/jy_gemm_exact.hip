@@ -598,7 +598,7 @@ static void gemm_exact(const Dev& W, int m, const float* A, float* C, int ldc, c
     const int ntiles = (W.rows + 63) / 64, T = gemm_form(GX_FORMS, m, ntiles);
     const int mt = (m + 4 * T - 1) / (4 * T), total = ntiles * mt;
 #define JY_GX(KERNEL) \
-    hipLaunchKernelGGL(KERNEL, dim3((unsigned)total), dim3(256), 0, st, W, m, mt, total, A, C, ldc, aux, (int)epi)
+    hipLaunchKernelGGL(KERNEL, dim3((unsigned)total), dim3(256), 0, st, W, m, mt, total, A, C, ldc, aux, (int)plain_epi(epi))
     switch (T) {
         case 16: JY_GX((gemm_exact_mm_kernel<Pieces, Dev, 16, 1>)); break;
         case 8: JY_GX((gemm_exact_mm_kernel<Pieces, Dev, 4, 2>)); break;
@@ -616,7 +616,7 @@ static void gemm_dense(const E* B, int K, int N, int m, const float* A, float* C
     const int T = sizeof(E) == 4 ? gemm_form(F32_FORMS, m, ntiles) : gemm_form(F16_FORMS, m, ntiles);
     const int mt = (m + 4 * T - 1) / (4 * T), total = ntiles * mt;
 #define JY_GD(KERNEL) \
-    hipLaunchKernelGGL(KERNEL, dim3((unsigned)total), dim3(256), 0, st, B, K, N, m, mt, total, A, C, ldc, aux, (int)epi)
+    hipLaunchKernelGGL(KERNEL, dim3((unsigned)total), dim3(256), 0, st, B, K, N, m, mt, total, A, C, ldc, aux, (int)plain_epi(epi))
     if constexpr (sizeof(E) == 2) {
         if (T == 1) {
             JY_GD((gemm_f16_exact_kernel<1>));

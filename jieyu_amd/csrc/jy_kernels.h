@@ -12,9 +12,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-namespace jy {
+#include "jy_epi.h"
 
-enum Epi { EPI_STORE = 0, EPI_BIAS = 1, EPI_RESID = 2, EPI_SWIGLU = 3, EPI_ROPE = 4, EPI_ARGMAX = 5 };
+namespace jy {
 
 struct Q8Dev {
     uint8_t* qs = nullptr;
@@ -133,8 +133,7 @@ int split_argmax_partials(int rows);
 size_t matvec_lds_bytes(int cols, bool norm);
 size_t matvec_lds_limit();
 // dense [K][N] matvec over the 64-column panel layout (f32, or f16 converted exactly),
-// fma chain over k per output column: EPI_STORE / EPI_BIAS / EPI_RESID, or
-// EPI_SWIGLU: out = silu(aux) * (W x)
+// fma chain over k per output column: EPI_STORE / EPI_BIAS / EPI_RESID
 void launch_matvec_f32(const float* B, int K, int N, const float* x, float* out, const float* aux, Epi epi,
                        hipStream_t st);
 void launch_matvec_f16(const uint16_t* B, int K, int N, const float* x, float* out, const float* aux, Epi epi,

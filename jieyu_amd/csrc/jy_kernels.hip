@@ -437,7 +437,7 @@ static DnSet<T> dense_set(const T* const* B, const int* N, float* const* out, co
 template <typename T>
 static void matvec_dense(const T* B, int K, int N, const float* x, float* out, const float* aux, Epi epi,
                          hipStream_t st) {
-    if (epi != EPI_BIAS) aux = nullptr;
+    if (plain_epi(epi) != EPI_BIAS) aux = nullptr;
     const DnSet<T> s = dense_set(&B, &N, &out, &aux, 1);
     if (epi == EPI_RESID)
         dense_launch<T, EPI_RESID, DN_PLAIN>(s, 1, K, x, nullptr, st);

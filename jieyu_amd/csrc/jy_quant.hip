@@ -526,6 +526,7 @@ bool launch_mv_gate_up(const DevW& gate, const DevW& up, const float* x, const f
 }
 
 void launch_mv(const DevW& W, const float* x, float* out, Epi epi, const float* aux, hipStream_t st) {
+    epi = plain_epi(epi);
     switch (W.type) {
         case JY_F32:
             launch_matvec_f32(static_cast<const float*>(W.dense), W.in, W.out, x, out, aux, epi, st);

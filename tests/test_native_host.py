@@ -51,3 +51,25 @@ def stage(tmp_path_factory):
 def test_pinned_ring(stage, case):
     r = subprocess.run([str(stage), case], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
+
+
+def test_plain_epilogues(tmp_path):
+    """the launches of plain products (store, bias, residual) refuse the other epilogues"""
+    src = tmp_path / "epi.cpp"
+    src.write_text("""
+#include "jy_epi.h"
+using namespace jy;
+static bool refused(Epi e) {
+    try { return plain_epi(e) != e; } catch (const std::exception&) { return true; }
+}
+int main() {
+    for (Epi e : {EPI_STORE, EPI_BIAS, EPI_RESID}) if (refused(e)) return 1;
+    for (Epi e : {EPI_SWIGLU, EPI_ROPE, EPI_ARGMAX}) if (!refused(e)) return 2;
+    return 0;
+}
+""")
+    compile_native(tmp_path / "epi", str(src))
+    assert subprocess.run([str(tmp_path / "epi")]).returncode == 0
+    # every one of them goes through that check
+    for f, n in (("jy_kernels.hip", 1), ("jy_gemm_exact.hip", 2), ("jy_quant.hip", 1)):
+        assert open(os.path.join(CSRC, f)).read().count("plain_epi(epi)") == n, f
