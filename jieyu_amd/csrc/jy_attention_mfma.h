@@ -5,7 +5,7 @@
 // int32 q.k dot, score = (float)dot * ((ks * qsc) * (1/sqrtf(hd))), weights e^(score - max);
 // the softmax sum and the p.v accumulation are reordered and the weights carried at 22 bits.
 //
-// Work split.  A workgroup of NW waves (4 or 8) takes one (kv head, slice of keys), and
+// Work split.  A workgroup of NW waves (4, 8 or, for prompt rows, 16) takes one (kv head, slice of keys), and
 // with DSP > 1 one tile of hd/DSP output dims over all the keys; wave w takes the slice's
 // steps w, w+NW, ... of 32 keys and keeps its own running (max, sum, o) per query head, with
 // no workgroup barrier in the key loop; the waves' results are merged through LDS at the end.

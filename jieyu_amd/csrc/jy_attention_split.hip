@@ -210,6 +210,21 @@ void launch_attention_whole(const AttnArgs& a, hipStream_t st) {
 // what their loads gain).  Per layer, 4 waves -> now: 61 rows x 5000 keys, Qwen2.5-7B heads
 // 50.2 -> 36.8 us (the keys and values through L2 at 9 TB/s), Llama-3-8B heads 54.6 -> 45.3; 61 x
 // 700 13.5 -> 11.2; 100 x 3000, Qwen2.5-0.5B heads 25.0 -> 18.0; 30 x 1000 11.8 -> 9.2.
+//
+// The waves' partial results are merged in wave order, so a row's last bits depend on the
+// waves, and with them on its chunk: the same row in a chunk of 61 over 5000 keys (16 waves)
+// and of 300 (4) agrees to about 5e-6 of its largest value, not bit for bit.
+static int split_cus() {
+    static const int n = [] {
+        int dev = 0, cus = 0;
+        return hipGetDevice(&dev) == hipSuccess &&
+                       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0
+                   ? cus
+                   : 256;
+    }();
+    return n;
+}
+
 template <int NW>
 static void prefill_launch(const AttnArgs& a, int R, hipStream_t st) {
     const dim3 grid(a.nkv, (a.nrows + R - 1) / R), block(64 * NW);
@@ -230,10 +245,10 @@ static void prefill_launch(const AttnArgs& a, int R, hipStream_t st) {
 void launch_attention_prefill_split(const AttnArgs& a, hipStream_t st) {
     const int R = SPL_GMAX / split_heads(a.nh / a.nkv);
     const long wgs = (long)a.nkv * ((a.nrows + R - 1) / R);
-    const int keys = a.start_pos + a.row0 + a.nrows;
-    if (wgs <= 256 && keys >= 2048)
+    const int keys = a.start_pos + a.row0 + a.nrows, cus = split_cus();
+    if (wgs <= cus && keys >= 2048)
         prefill_launch<16>(a, R, st);
-    else if (wgs <= 512 && keys >= 512)
+    else if (wgs <= 2 * cus && keys >= 512)
         prefill_launch<8>(a, R, st);
     else
         prefill_launch<4>(a, R, st);
