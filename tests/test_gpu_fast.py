@@ -177,6 +177,32 @@ def test_mfma_gemm_tiles(jy, oracle_lib, m, rows, cols):
     assert np.all(np.abs(got - A64 @ wf.T) <= bound)
 
 
+# (digests taken from the 16x16x32 form of the kernel that read weights and activations through
+# LDS; integers and powers of two, so the inputs are the same everywhere)
+@pytest.mark.parametrize("m,rows,cols,digest", [
+    (2, 77, 32, "1c5d4d33d3330ef4"), (31, 130, 96, "8b3cfa93b7e55694"), (33, 1152, 896, "7c4bbdd63f4b3937"),
+    (61, 4096, 4096, "007a84c2da651963"), (61, 28679, 160, "c62caab01bfa4a03"), (100, 896, 4864, "f204319c4746fbc6"),
+    (129, 4112, 1056, "1f76bfbeffc81af3"), (200, 6144, 512, "8e0108bf3aca763e"), (300, 20011, 224, "f6ab50e33dd2ab01"),
+    (509, 9728, 896, "376a7c3b8be825a7"), (1000, 12007, 96, "4e10e2623135bb12"), (1024, 4112, 1056, "e8bba849f7315560"),
+    (40, 1000, 17024, "5df0beab876ece5f")])
+def test_mfma_gemm_keeps_its_bits(jy, m, rows, cols, digest):
+    """another tile or K slice order would be within the tolerance, and still move where a long
+    greedy run leaves the reference: the sums' bits stay what they were"""
+    import hashlib
+    say(f"mfma gemm bits m={m} {rows}x{cols}")
+    rng = np.random.default_rng(m * rows + cols)
+    w = np.zeros((rows, cols // 32, 34), np.uint8)
+    w[:, :, 2:] = rng.integers(-127, 128, (rows, cols // 32, 32)).astype(np.int8).view(np.uint8)
+    d = (rng.integers(128, 1024, (rows, cols // 32, 1)) * 2.0 ** -17).astype(np.float16)
+    w[:, :, :2] = d.view(np.uint8).reshape(rows, cols // 32, 2)
+    A = (rng.integers(-2 ** 20, 2 ** 20, (m, cols)) * 2.0 ** -18).astype(np.float32)
+    M = jy.Q8Matrix(w.reshape(-1), rows, cols)
+    M.set_mode(jy.MODE_MFMA_PREFILL)
+    got = M.gemm(A)
+    M.close()
+    assert hashlib.sha256(got.tobytes()).hexdigest()[:16] == digest
+
+
 def attention_alone(olib, heads, kv, hd):
     """a one-layer Q8_0 model whose layer output minus its input is the attention's output: Wo the
     identity, the MLP zero; scores of standard deviation about 0.4.  (desc, what it points to, Wq, Wk, Wv)"""
