@@ -233,8 +233,9 @@ __global__ __launch_bounds__(256) void gemm_exact_kernel(Dev W, int m, int mt, i
 //
 // v_mfma_f32_{16x16x1_4b, 4x4x1_16b} with a zero addend is an outer product whose values are
 // each rounded once, as a multiply's are (subnormals, infinities and all): TT tokens x 64
-// columns (one per lane of B) of one k per instruction, the matrix cores running beside the
-// vector unit, which is left with the add.  One register of A holds 64 / TT k of the TT
+// columns (one per lane of B) of one k per instruction, and the vector unit adds it to the
+// sums.  The product takes the vector unit's time all the same (at the top); what is gained are the
+// activations, 16 bytes per lane instead of scalar loads.  One register of A holds 64 / TT k of the TT
 // tokens (lane TT j + t: token t), of which the instruction's broadcast picks one (ABID j).
 
 template <int TT> struct Outer;
@@ -285,8 +286,10 @@ __device__ __forceinline__ void outer_store(const typename Outer<TT>::vec (&acc)
 }
 
 // (registers for three or four workgroups per CU: a lone wave issues a vector instruction per
-// 2.05 ns, two or more waves of a SIMD together one per 0.94.  The packed pieces of the next chunk replace this one's once its last step is staged,
-// and the activations are reloaded piece by piece as they are used up)
+// 2.05 ns, two or more waves of a SIMD together one per 0.94.  The packed pieces of the next chunk
+// replace this one's once its last step is staged, and the activations are reloaded piece by piece
+// as they are used up.  Within those registers the 16-token form spills 2 (Q8_0), 6 (Q4_K), 25
+// (Q5_K) and 23 (Q6_K), the 8-token form 4 (Q5_K) and 6 (Q6_K) registers.)
 template <class Pieces, class Dev, int TT, int MT>
 __global__ __launch_bounds__(256, TT == 16 ? 3 : 4) void gemm_exact_mm_kernel(
     Dev W, int m, int mt, int total, const float* __restrict__ A, float* __restrict__ C, int ldc,
@@ -565,7 +568,8 @@ hipError_t gemm_exact_init() {
 // A form's time per k in ns when the busiest CU has c workgroups of its grid: `one` at least,
 // else slope c + off.  Measured with 4096 x 4096, 4096 x 14336, 6144 x 4096 and 28672 x 4096
 // weights at 61, 130 and 200 rows (quantized: Q8_0), and with K x N of 512 x 1376, 2048 x 5632,
-// 5632 x 2048, 896 x 4864 and others at 8 to 200 rows (dense); the fit is within 15 %.
+// 5632 x 2048, 896 x 4864 and others at 8 to 200 rows (dense); the fit is within 15 %.  The k-quants
+// take Q8_0's table: their own times, with more unpacking and the spills above, were not fitted.
 struct GemmForm {
     int T;
     float one, slope, off;

@@ -4,8 +4,8 @@
 //
 // Numbers.  The int8 weights are exact in fp16.  Each activation row is scaled by a power
 // of two that puts its largest magnitude in [2^13, 2^14) and split into an fp16 high part
-// and an fp16 low part (the rounding remainder), 22 significant bits together.  One
-// v_mfma_f32_16x16x32_f16 per part gives a 32-weight block's sum sum_k a[k] q[k] in fp32
+// and an fp16 low part (the rounding remainder), 22 significant bits together.  Two
+// v_mfma_f32_32x32x16_f16 per part give a 32-weight block's sum sum_k a[k] q[k] in fp32
 // (every product exact, fp32 additions); the block's fp16 scale multiplies that sum in an
 // fp32 fma into the running result, and the epilogue undoes the row's power of two.  So
 // the differences from the reference's fp32 loop are the order of the fp32 additions and
