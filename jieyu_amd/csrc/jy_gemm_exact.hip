@@ -19,8 +19,8 @@
 // 14 ns per SIMD, their 16 adds 17 ns, both together 30; 16 multiplies and adds 29 with two
 // waves per SIMD), so the gain is the loads', not the arithmetic's.  T and the form are chosen
 // per launch (gemm_form) from times measured per k.
-// Llama-3-8B Q8_0, 200 rows, before (vector unit only) -> now: gate/up 28672 x 4096 1352 -> 1000 us,
-// QKV 6144 x 4096 380 -> 280, O 4096 x 4096 308 -> 210, down 4096 x 14336 1010 -> 700.
+// Llama-3-8B Q8_0, 200 rows, 64 x 64 tiles through LDS -> now (both builds in turn): gate/up 28672 x
+// 4096 1423 -> 1072 us, QKV 6144 x 4096 577 -> 302, O 4096 x 4096 560 -> 226, down 4096 x 14336 1912 -> 765.
 #include <algorithm>
 #include <type_traits>
 
