@@ -280,7 +280,10 @@ struct KqMats {
     int row0[3];  // first output row of each matrix
 };
 
-// One matrix by `nwg` workgroups of 4 waves: wave w takes row groups w, w + 4 nwg, ...
+// One matrix by `nwg` workgroups of 4 waves.  With the norm (NV > 0) wave w takes row groups w, w +
+// 4 nwg, ..., the loads running ahead across them; without, one row group, and with NV = KQ_SHORT
+// a row of at most U chunks, one buffer.
+static constexpr int KQ_SHORT = -1;
 template <int TYPE, int EPI, int NV, int U>
 __device__ __forceinline__ void kq_body(const KQDev& W, int wg, int nwg, int row0, const float* __restrict__ x,
                                         const float* __restrict__ nw, float* __restrict__ out, const MvArgs& a,
@@ -301,7 +304,6 @@ __device__ __forceinline__ void kq_body(const KQDev& W, int wg, int nwg, int row
     };
     kq_stage<NV, U>(x, nw, W.cols, XS, xs, red, [&]() {
         load(A);
-        if (NV == 0) load(B);
     });
     if (NV > 0) load(B);
     const float* xrow = xs + g * XS;
@@ -319,6 +321,24 @@ __device__ __forceinline__ void kq_body(const KQDev& W, int wg, int nwg, int row
         }
     };
     const int nb = (nsb + U - 1) / U;  // buffers per row group
+    if constexpr (NV <= 0) {
+        if (wid >= W.groups) return;
+        const int lr = wid * 4 + r, row = row0 + lr;
+        const bool own = g == 0 && lr < W.rows;
+        const MvPre pre = mv_preload<EPI>(row, own, r, a, out);
+        if constexpr (NV == KQ_SHORT) {
+            compute(A, 0);
+        } else {
+            for (int s0 = 0; s0 < nsb; s0 += 2 * U) {
+                B.load(W, wid, s0 + U, lane, r);
+                compute(A, s0);
+                if (s0 + 2 * U < nsb) A.load(W, wid, s0 + 2 * U, lane, r);
+                compute(B, s0 + U);
+            }
+        }
+        mv_epilogue<EPI>(kq_tree(a0, a1), row, own, r, row0 + W.rows, a, out, bv, bi, &pre);
+        return;
+    }
     bool cur_b = false;                // whether the next buffer to compute is B
     for (int rg = wid; rg < W.groups; rg += TW) {
         const int lr = rg * 4 + r, row = row0 + lr;
@@ -346,10 +366,12 @@ __device__ __forceinline__ void kq_body(const KQDev& W, int wg, int nwg, int row
     }
 }
 
-// The decode matvec.  What bounds it: at 1024 row groups (one wave per SIMD) the latency of
-// the weight stream, so U is 8 chunks a buffer there (16 in flight per wave) and 4 otherwise;
-// past that the dequantisation (about 90 VALU instructions per 256 weights of 4 rows).  The
-// vector used to be staged by a loop of dependent 4-byte loads before the first weight load.
+// The decode matvec.  What bounds it: at few row groups (1024: one wave per SIMD) the latency of
+// the weight stream; past that the dequantisation (about 90 VALU instructions per 256 weights of
+// 4 rows).  The vector is staged with its loads ahead of the first weights' (dependent 4-byte loads
+// before them: 4096 x 14336 30.5 us).  Without the norm a wave takes one row group: running the loads
+// ahead across row groups there cost 0.3 to 0.9 us a launch in buffers read and never used (1024 x 4096
+// 7.6 against 6.7).
 template <int EPI, int NV, int U>
 __global__ __launch_bounds__(256, U == 4 && NV <= 4 ? 4 : 2) void matvec_kq_kernel(KqMats M, const float* __restrict__ x,
                                                         const float* __restrict__ nw, float* __restrict__ out,
@@ -459,14 +481,24 @@ static KqMats kq_mats(const KQDev* const* W, int n) {
     return M;
 }
 
+// Rows of up to 4 chunks (1024 inputs) take one buffer: 64 x 256 2.5 us against 2.9 in the loop.  Eight
+// chunks a buffer pay for long rows alone, with at most a workgroup per CU: Q4_K 4096 x 14336 19.5 ->
+// 18.7 us, but 2048 x 5632 8.6 -> 9.1, 1024 x 3072 5.7 -> 5.9, 2048 x 2048 4.4 -> 5.5.
 template <int EPI, int NV>
 static void mv_kq(const KqMats& M, const float* x, const float* nw, float* out, const MvArgs& a, hipStream_t st) {
     const dim3 grid((unsigned)M.wg0[3]), block(256);
     const size_t lds = mv_kq_lds_bytes(M.W[0].cols);
-    if (M.wg0[3] <= g_kq_cus)
-        hipLaunchKernelGGL((matvec_kq_kernel<EPI, NV, 8>), grid, block, lds, st, M, x, nw, out, a);
-    else
-        hipLaunchKernelGGL((matvec_kq_kernel<EPI, NV, 4>), grid, block, lds, st, M, x, nw, out, a);
+    if constexpr (NV == 0) {
+        if (M.W[0].nsb <= 4) {
+            hipLaunchKernelGGL((matvec_kq_kernel<EPI, KQ_SHORT, 4>), grid, block, lds, st, M, x, nw, out, a);
+            return;
+        }
+        if (M.wg0[3] <= g_kq_cus && M.W[0].nsb > 32) {
+            hipLaunchKernelGGL((matvec_kq_kernel<EPI, 0, 8>), grid, block, lds, st, M, x, nw, out, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((matvec_kq_kernel<EPI, NV, 4>), grid, block, lds, st, M, x, nw, out, a);
 }
 
 static bool is_kq(const DevW& w) { return w.type == JY_Q4_K || w.type == JY_Q5_K || w.type == JY_Q6_K; }
@@ -474,7 +506,8 @@ static bool is_kq(const DevW& w) { return w.type == JY_Q4_K || w.type == JY_Q5_K
 static void mv_kq1(const DevW& W, const float* x, const float* nw, float* out, Epi epi, const float* aux,
                    hipStream_t st) {
     const KQDev* w[1] = {&W.kq};
-    const KqMats M = kq_mats(w, 1);
+    KqMats M = kq_mats(w, 1);
+    if (!nw) M.wg0[1] = M.wg0[2] = M.wg0[3] = (W.kq.groups + 3) / 4;
     MvArgs a;
     a.aux = aux;
     if (nw) {
@@ -549,18 +582,17 @@ hipError_t quant_init() {
     if (e == hipSuccess && cus > 0) g_kq_cus = cus;
     for (const void* f : {reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, 0, 4>),
                           reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, 0, 8>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, KQ_SHORT, 4>),
                           reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, 4, 4>),
-                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, 4, 8>),
                           reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, 8, 4>),
-                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_STORE, 8, 8>),
                           reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_BIAS, 0, 4>),
                           reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_BIAS, 0, 8>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_BIAS, KQ_SHORT, 4>),
                           reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_RESID, 0, 4>),
                           reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_RESID, 0, 8>),
+                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_RESID, KQ_SHORT, 4>),
                           reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_ROPE, 4, 4>),
-                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_ROPE, 4, 8>),
                           reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_ROPE, 8, 4>),
-                          reinterpret_cast<const void*>(&matvec_kq_kernel<EPI_ROPE, 8, 8>),
                           reinterpret_cast<const void*>(&matvec_kq_pair_kernel<JY_Q4_K, 4>),
                           reinterpret_cast<const void*>(&matvec_kq_pair_kernel<JY_Q4_K, 8>),
                           reinterpret_cast<const void*>(&matvec_kq_pair_kernel<JY_Q5_K, 4>),

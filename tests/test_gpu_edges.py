@@ -136,6 +136,16 @@ def check_generate(jy, oracle_lib, spec):
     assert bits_equal(logits, wl)
 
 
+# the k-quant matvec alone: rows of one buffer (up to 1024 inputs), of a remainder of the two
+# buffers' 8 or 16 chunks, either side of the longer buffers' 8192 inputs; row groups cut short, and
+# more than a workgroup per CU
+@pytest.mark.parametrize("t", [QM.JY_Q4_K, QM.JY_Q5_K, QM.JY_Q6_K])
+@pytest.mark.parametrize("n,k", [(1, 256), (66, 768), (4103, 1024), (13, 1280), (130, 2048), (5, 2304), (67, 3328),
+                                 (17000, 512), (4100, 4352), (9, 8192), (18, 8448), (4098, 8448), (1030, 14336)])
+def test_kquant_matvec_widths(jy, oracle_lib, t, n, k):
+    check_exact_gemm(jy, oracle_lib, t, n, k, 1)
+
+
 # dense decode: the launches with RMSNorm (q/k/v, gate/up, the head) and with SiLU (down) at input
 # widths under, at and over one block of the panel (256 f32, 512 f16 rows), not a multiple of a
 # 16-byte piece, at and past the widest row the launch holds (6144), outputs that cut a panel,
