@@ -328,8 +328,10 @@ __global__ __launch_bounds__(DN_THREADS) void matvec_dense_kernel(DnSet<T> set, 
     // flight).
     auto chains = [&](int b) {
         if (wave != 0) return;
-        // (32 steps per group, f32 and f16 alike)
-        constexpr int G = 32 / PER, NP = RB / PER, XQ = PER / 4;
+        // (pieces per group: 4, and 8 for f32 in the launches of a layer's norm and SiLU, where the
+        // tiny model's 24 tokens take 5740 us against 5780.  The plain matvec loses by 8: the first
+        // group of each block is read cold, 4096 x 14336 78.3 -> 81.2 us, 2048 x 5632 32.7 -> 33.8)
+        constexpr int G = XF == DN_PLAIN ? 4 : 32 / PER, NP = RB / PER, XQ = PER / 4;
         const int rem = nkb - b * NP;
         const int ns = rem < NP ? (rem + G - 1) / G * G : NP;
         const uint4* col = tile + (b & 1) * PIECES + lane;
