@@ -132,7 +132,8 @@ JYHIP_API int jyhip_forward_cached_to(jyhip_model* model, jyhip_kv* kv, const fl
  * copies X from and back to the host and waits for the model's stream, so it cannot be
  * recorded into a caller's HIP graph: it allocates nothing, it is not capturable.  The
  * calling thread copies the rows itself, and nothing is allocated on the host for them (they
- * go through the model's pinned ring once a jyhip_forward_cached call has made it).
+ * go through the model's pinned memory once a jyhip_forward_cached call of as many rows has
+ * made it).
  * Same arguments, checks and results as jyhip_forward_cached with layer_out == NULL.
  * Its workspace is one static array of JYHIP_NOALLOC_SCRATCH_BYTES in each GPU's memory,
  * held until the process ends; a call whose rows and keys need more (a long prompt, a

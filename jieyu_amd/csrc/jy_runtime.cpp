@@ -1599,7 +1599,7 @@ int generate_impl(jyhip_model* m, jyhip_kv* kv_in, const int* prompt, int plen, 
 // by the model's first such call, and helper threads for many rows)
 void rows_in(jyhip_model* m, Workspace& w, const float* X, int seq, bool alloc) {
     const size_t n = sizeof(float) * seq * m->H;
-    if (m->stage.ready(alloc))
+    if (m->stage.ready(n, alloc))
         CK(m->stage.to_device(w.X, X, n, m->stream, alloc));
     else
         CK(hipMemcpyAsync(w.X, X, n, hipMemcpyHostToDevice, m->stream));
@@ -1608,7 +1608,7 @@ void rows_in(jyhip_model* m, Workspace& w, const float* X, int seq, bool alloc) 
 void rows_out(jyhip_model* m, Workspace& w, float* out, int seq, bool alloc) {
     hipStream_t st = m->stream;
     const size_t row = sizeof(float) * m->H;
-    if (m->stage.ready(alloc)) {  // the norm writes the pinned ring itself
+    if (m->stage.ready(row * seq, alloc)) {  // the norm writes the pinned ring itself
         const auto norm = [&](size_t r0, size_t n, void* p) {
             launch_rmsnorm(w.X + r0 * m->H, static_cast<float*>(p), m->final_rms, m->H, (int)n, st);
         };

@@ -95,12 +95,22 @@ class Team {
 
 }  // namespace
 
-bool HostStage::ready(bool create) {
-    if (!ring_ && create && !tried_) {
-        tried_ = true;
-        return init();
+bool HostStage::ready(size_t n, bool create) {
+    if (ring_) return true;
+    if (n <= SMALL) {
+        if (!small_ && create && !tried_small_) {
+            tried_small_ = true;
+            void* p = nullptr;
+            if (hipHostMalloc(&p, SMALL, hipHostMallocDefault) == hipSuccess)
+                small_ = static_cast<unsigned char*>(p);
+            else
+                (void)hipGetLastError();
+        }
+        return small_ != nullptr;
     }
-    return ring_ != nullptr;
+    if (!create || tried_) return false;
+    tried_ = true;
+    return init();
 }
 
 bool HostStage::init() {
@@ -109,19 +119,25 @@ bool HostStage::init() {
     ring_ = ok ? static_cast<unsigned char*>(p) : nullptr;
     for (int i = 0; ok && i < SLOTS; i++) ok = hipEventCreateWithFlags(&ev_[i], hipEventDisableTiming) == hipSuccess;
     if (!ok) {
-        release();
+        free_ring();
         (void)hipGetLastError();
     }
     return ok;
 }
 
-void HostStage::release() {
+void HostStage::free_ring() {
     for (hipEvent_t& e : ev_) {
         if (e) (void)hipEventDestroy(e);
         e = nullptr;
     }
     if (ring_) (void)hipHostFree(ring_);
     ring_ = nullptr;
+}
+
+void HostStage::release() {
+    free_ring();
+    if (small_) (void)hipHostFree(small_);
+    small_ = nullptr;
 }
 
 // the ring free of an earlier transfer that ended in an error
@@ -140,8 +156,8 @@ hipError_t HostStage::to_device(void* dst, const void* src, size_t n, hipStream_
     auto* d = static_cast<unsigned char*>(dst);
     auto* s = static_cast<const unsigned char*>(src);
     if (nch == 1) {
-        memcpy(ring_, s, n);
-        launch_copy(ring_, d, n, st);
+        memcpy(one(), s, n);
+        launch_copy(one(), d, n, st);
         return hipGetLastError();
     }
     auto copy = [&](size_t c, size_t off, size_t len) {
@@ -184,10 +200,10 @@ hipError_t HostStage::to_host(void* dst, size_t rows, size_t row_bytes, hipStrea
     auto* d = static_cast<unsigned char*>(dst);
     // (the slots' copies to the GPU are ahead of the producers on the stream)
     if (nch == 1) {
-        produce(0, rows, ring_);
+        produce(0, rows, one());
         if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(st)) != hipSuccess) return e;
         busy_ = false;
-        memcpy(d, ring_, rows * row_bytes);
+        memcpy(d, one(), rows * row_bytes);
         return hipSuccess;
     }
     auto copy = [&](size_t c, size_t off, size_t len) {

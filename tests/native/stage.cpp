@@ -35,6 +35,7 @@ static long round_trip(HostStage& s, size_t rows, size_t row, bool threads, uint
     fill(src, seed);
     const std::vector<uint32_t> keep = src;
     uint32_t* d = dev.data();
+    CHECK(s.ready(4 * src.size(), false));
     const long before = g_news;
     CHECK(s.to_device(d, src.data(), 4 * src.size(), nullptr, threads) == hipSuccess);
     for (uint32_t& x : src) x = 0;  // (it may be reused at once)
@@ -61,11 +62,22 @@ static const size_t SIZES[][2] = {{1, 1},      {3, 5},      {1, 4096},    {33, 4
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     HostStage s;
+    const size_t few = HostStage::SMALL, more = HostStage::SMALL + 4;
     if (!strcmp(what, "made_when_needed")) {
-        CHECK(!s.ready(false) && hip_stub::g_host_allocs == 0);
-        CHECK(s.ready(true) && s.ready(false) && s.ready(true) && hip_stub::g_host_allocs == 1);
+        CHECK(!s.ready(4, false) && !s.ready(more, false) && hip_stub::g_host_allocs == 0);
+        CHECK(s.ready(few, true) && s.ready(4, false) && s.ready(few, true) && hip_stub::g_host_allocs == 1);
+        CHECK(!s.ready(more, false) && hip_stub::g_live_events == 0);
+        for (const auto& z : SIZES)
+            if (4 * z[0] * z[1] <= few) round_trip(s, z[0], z[1], true, 9);
+        CHECK(s.ready(more, true) && s.ready(more, false) && s.ready(4, true) && hip_stub::g_host_allocs == 2);
+        for (const auto& z : SIZES) round_trip(s, z[0], z[1], true, 9);
         s.release();
-        CHECK(hip_stub::g_host_frees == 1);
+        CHECK(hip_stub::g_host_frees == 2 && hip_stub::g_live_events == 0);
+        // the ring first: nothing else is needed
+        HostStage r;
+        CHECK(r.ready(more, true) && r.ready(4, true) && hip_stub::g_host_allocs == 3);
+        for (const auto& z : SIZES) round_trip(r, z[0], z[1], true, 9);
+        r.release();
         // no pinned memory, or no k-th event: no ring, nothing left behind, no second try
         for (int k = 0; k <= HostStage::SLOTS; k++) {
             HostStage f;
@@ -73,16 +85,34 @@ int main(int argc, char** argv) {
             hip_stub::g_fail_event_at = k;
             hip_stub::g_events = 0;
             const int before = hip_stub::g_host_allocs;
-            CHECK(!f.ready(true));
+            CHECK(!f.ready(more, true));
+            if (k == 0) CHECK(!f.ready(few, true));
             hip_stub::g_fail_host_malloc = hip_stub::g_fail_event_at = 0;
-            CHECK(!f.ready(true) && !f.ready(false));
+            CHECK(!f.ready(more, true) && !f.ready(more, false));
+            if (k == 0) CHECK(!f.ready(few, true) && !f.ready(few, false));
             CHECK(hip_stub::g_host_allocs == before + (k != 0) && hip_stub::g_host_allocs == hip_stub::g_host_frees);
             CHECK(hip_stub::g_live_events == 0);
+            if (k != 0) {  // (few rows still have their buffer)
+                CHECK(f.ready(few, true));
+                round_trip(f, 3, 5, true, 9);
+            }
             f.release();
         }
+        CHECK(hip_stub::g_host_allocs == hip_stub::g_host_frees);
         return 0;
     }
-    CHECK(s.ready(true));
+    if (!strcmp(what, "after_an_error")) {  // few rows in, no rows out, then more
+        CHECK(s.ready(few, true));
+        std::vector<uint32_t> a(few / 4), da(few / 4), b(more / 4), db(more / 4);
+        fill(a, 1);
+        fill(b, 2);
+        CHECK(s.to_device(da.data(), a.data(), few, nullptr, true) == hipSuccess);
+        CHECK(s.ready(more, true));
+        CHECK(s.to_device(db.data(), b.data(), more, nullptr, true) == hipSuccess);
+        hipStreamSynchronize(nullptr);
+        CHECK(da == a && db == b);
+    }
+    CHECK(s.ready(more, true));
     if (!strcmp(what, "round_trip")) {
         for (int pass = 0; pass < 3; pass++)
             for (const auto& z : SIZES) round_trip(s, z[0], z[1], pass != 1, 17 * pass + 1);
